@@ -28,3 +28,13 @@ def gpu():
     import eigen_amd
     eigen_amd.lib()  # must load: no fallback
     return True
+
+
+def pytest_collection_modifyitems(items):
+    # these call the reference built from its sources (oracle/Makefile), which
+    # exists only where those sources do
+    from oracle import pyoracle
+    if pyoracle.ref() is None:
+        for item in items:
+            if item.name.startswith("test_dgetrf_rectangular"):
+                item.add_marker(pytest.mark.skip(reason="oracle/_ref is not built"))
