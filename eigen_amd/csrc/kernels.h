@@ -90,6 +90,9 @@ template <typename T>
 int trsv_device(eamd_handle* h, int n, const T* A, int64_t lda, bool rowmajor, bool lower,
                 bool unit, T* X, int64_t ldx, int nrhs);
 int trsv_check_error(eamd_handle* h);
+// the same for many right-hand sides, on matrix products (trsm.hip)
+int trsm_blocked(eamd_handle* h, int n, const double* A, int64_t lda, bool rowmajor, bool lower,
+                 bool unit, double* X, int64_t ldx, int nrhs);
 // X <- P X (forward) or P^T X with P given as a transposition sequence
 template <typename T>
 int apply_transpositions(eamd_handle* h, int n, const int* t, bool forward, T* X, int64_t ldx,

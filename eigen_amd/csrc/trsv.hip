@@ -1,9 +1,9 @@
-// trsv.hip -- blocked triangular solves with few right-hand sides.
+// trsv.hip -- blocked triangular solves with one right-hand side.
 //
 // Replaces triangular_solve_vector (TriangularSolverVector.h:88-139) and the
-// few-RHS use of triangular_solve_matrix (TriangularSolverMatrix.h:38-184)
+// one-column use of triangular_solve_matrix (TriangularSolverMatrix.h:38-184)
 // inside PartialPivLU::_solve_impl (PartialPivLU.h:226-244) and
-// LLT::_solve_impl (LLT.h:475-505).
+// LLT::_solve_impl (LLT.h:475-505); several columns go to trsm.hip.
 //
 // One workgroup per BS-row block, dispatched in dependency order.  Workgroup
 // b first inverts its diagonal block in LDS (independent of the others, so
@@ -13,8 +13,6 @@
 // epoch (an aligned 8-byte store is single-copy atomic, so a word with the
 // right epoch has the right payload): consumers poll the words themselves,
 // with no flag and no cache write-back or invalidate on the critical path.
-// Several right-hand sides run as up to four independent chains of four
-// columns in one launch, their workgroups interleaved block by block.
 #include <algorithm>
 
 #include "common.h"
@@ -46,45 +44,36 @@ struct XWords {
   static constexpr int n = sizeof(T) / 4;  // 32-bit payload words per value
 };
 
-template <typename T, bool ROWMAJOR, bool LOWER, bool UNIT, int BS, int NRC>
+template <typename T, bool ROWMAJOR, bool LOWER, bool UNIT, int BS>
 __global__ __launch_bounds__(4 * BS) void trsv_chain_kernel(int n, const T* __restrict__ A,
                                                          int64_t lda, T* __restrict__ X,
-                                                         int64_t ldx, int c0, int nrhs,
                                                          u64* __restrict__ xw, unsigned epoch,
-                                                         int* __restrict__ err, int nch,
-                                                         int spin_limit) {
-  static_assert((BS == 64 || BS == 128) && (NRC == 16 || NRC == 4 || NRC == 1),
-                "four threads per row of a 64- or 128-row block");
+                                                         int* __restrict__ err, int spin_limit) {
+  static_assert(BS == 64 || BS == 128, "four threads per row of a 64- or 128-row block");
   constexpr int NT = 4 * BS;   // threads
   constexpr int SEG = BS / 4;  // columns of a predecessor block per thread
   constexpr int NW = XWords<T>::n;
-  constexpr int CHUNK = BS * NRC * NW;          // words of one block's solution
+  constexpr int CHUNK = BS * NW;                // words of one block's solution
   constexpr int WPT = (CHUNK + NT - 1) / NT;    // words staged per thread
   __shared__ T Dinv[BS][BS + 1];
   __shared__ T Tb[BS][BS + 1];
-  __shared__ T accs[BS][NRC];
+  __shared__ T accs[BS];
   __shared__ unsigned xsw[2][CHUNK];  // staged solution of the current predecessor
   __shared__ int s_abort;
-  // FP32, one right-hand side: M = inv(T_bb) T_bl for the last predecessor l
+  // FP32: M = inv(T_bb) T_bl for the last predecessor l
   // is formed while the block waits, and inv(T_bb) (B_b - sum over the other
   // predecessors) before l's solution arrives, so the step after it is one
   // row of M times X_l (one barrier instead of two, no reduction through LDS)
-  constexpr bool kM = NRC == 1 && sizeof(T) == 4;
+  constexpr bool kM = sizeof(T) == 4;
   __shared__ T Tl[kM ? BS : 1][BS + 1];
   __shared__ unsigned xwv[kM ? NT / 64 : 1][BS];  // (kM) each wave's copy of X_l
   const int tid = threadIdx.x;
   const int nblk = (n + BS - 1) / BS;
-  // nch independent chains of NRC columns each, interleaved block by block
-  // (workgroup w * nch + k is block w of chain k: every chain's blocks are
-  // dispatched in dependency order), each with its own exchange words
-  const int chain = blockIdx.x % nch;
-  const int w = blockIdx.x / nch;
-  c0 += chain * NRC;
-  xw += (size_t)chain * nblk * BS * NRC * NW;
+  // workgroups are dispatched in dependency order
+  const int w = blockIdx.x;
   const int b = LOWER ? w : nblk - 1 - w;
   const int rb0 = b * BS;
   const int bs = min(BS, n - rb0);
-  const int nc = min(NRC, nrhs - c0);
   const int r = tid >> 2, q = tid & 3;  // my row of the block, my quarter of each column block
   const int ndep = LOWER ? b : nblk - 1 - b;
   const int jl = LOWER ? b - 1 : b + 1;  // the last predecessor (ndep > 0)
@@ -145,18 +134,13 @@ __global__ __launch_bounds__(4 * BS) void trsv_chain_kernel(int n, const T* __re
       }
     }
   }
-  T acc[NRC];
-#pragma unroll
-  for (int c = 0; c < NRC; ++c) acc[c] = T(0);
+  T acc = T(0);
   // predecessors taken in the loop (kM: all but the last)
   const int nloop = kM ? max(ndep - 1, 0) : ndep;
   const bool rvalid = r < bs;
-  // the block's right-hand sides, requested now: read after the loop they
-  // would put a memory round trip on every link of the chain
-  T bval[NRC];
-#pragma unroll
-  for (int c = 0; c < NRC; ++c)
-    bval[c] = (q == 0 && rvalid && c < nc) ? X[(int64_t)(c0 + c) * ldx + rb0 + r] : T(0);
+  // the block's right-hand side, requested now: read after the loop it would
+  // put a memory round trip on every link of the chain
+  const T bval = (q == 0 && rvalid) ? X[rb0 + r] : T(0);
   // a row-major segment is contiguous: 16-byte loads when aligned (a quarter
   // or half of the address work of element loads, which the CU's address
   // unit otherwise limits)
@@ -195,7 +179,7 @@ __global__ __launch_bounds__(4 * BS) void trsv_chain_kernel(int n, const T* __re
   auto stage = [&](int d) {
     const int jb = LOWER ? d : nblk - 1 - d;
     const int par = d & 1;
-    // my words of the predecessor's solution (row jr, column c, half h): all
+    // my words of the predecessor's solution (row, half): all
     // loads in flight together, then only the words not yet published are
     // read again
     const u64* wsrc[WPT];
@@ -204,10 +188,9 @@ __global__ __launch_bounds__(4 * BS) void trsv_chain_kernel(int n, const T* __re
 #pragma unroll
     for (int k = 0; k < WPT; ++k) {
       const int widx = tid + k * NT;
-      const int row = jb * BS + widx / (NRC * NW);
-      const int c = (widx / NW) % NRC;
-      need[k] = widx < CHUNK && row < n && c < nc;
-      wsrc[k] = xw + (size_t)row * NRC * NW + (widx % (NRC * NW));
+      const int row = jb * BS + widx / NW;
+      need[k] = widx < CHUNK && row < n;
+      wsrc[k] = xw + (size_t)row * NW + widx % NW;
       wv[k] = need[k] ? __hip_atomic_load(const_cast<u64*>(wsrc[k]), __ATOMIC_RELAXED,
                                           __HIP_MEMORY_SCOPE_AGENT)
                       : 0ull;
@@ -254,23 +237,18 @@ __global__ __launch_bounds__(4 * BS) void trsv_chain_kernel(int n, const T* __re
     stage(d);
     if (bad) break;
     const int cb = jb * BS + q * SEG;
+    T sum = T(0);
 #pragma unroll
-    for (int c = 0; c < NRC; ++c) {
-      if (c < nc) {
-        T sum = T(0);
-#pragma unroll
-        for (int i = 0; i < SEG; ++i) {
-          const unsigned* wp = &xsw[par][((q * SEG + i) * NRC + c) * NW];
-          T xv;
-          if (NW == 2)
-            xv = (T)__longlong_as_double((long long)(((u64)wp[1] << 32) | wp[0]));
-          else
-            xv = (T)__uint_as_float(wp[0]);
-          if (cb + i < n) sum += tcur[i] * xv;
-        }
-        acc[c] += sum;
-      }
+    for (int i = 0; i < SEG; ++i) {
+      const unsigned* wp = &xsw[par][(q * SEG + i) * NW];
+      T xv;
+      if (NW == 2)
+        xv = (T)__longlong_as_double((long long)(((u64)wp[1] << 32) | wp[0]));
+      else
+        xv = (T)__uint_as_float(wp[0]);
+      if (cb + i < n) sum += tcur[i] * xv;
     }
+    acc += sum;
 #pragma unroll
     for (int i = 0; i < SEG; ++i) tcur[i] = tnext[i];
   }
@@ -279,32 +257,17 @@ __global__ __launch_bounds__(4 * BS) void trsv_chain_kernel(int n, const T* __re
     __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   // the four quarters of a row sit in lanes 4r .. 4r+3 of one wave
-#pragma unroll
-  for (int c = 0; c < NRC; ++c) {
-    acc[c] += __shfl_xor(acc[c], 1);
-    acc[c] += __shfl_xor(acc[c], 2);
-  }
-  if (q == 0) {
-#pragma unroll
-    for (int c = 0; c < NRC; ++c)
-      accs[r][c] = (rvalid && c < nc) ? bval[c] - acc[c] : T(0);
-  }
+  acc += __shfl_xor(acc, 1);
+  acc += __shfl_xor(acc, 2);
+  if (q == 0) accs[r] = rvalid ? bval - acc : T(0);
   __syncthreads();
   if (s_abort) return;
   // ---- X_b = inv(T_bb) * (B_b - sum): thread (r, q) takes a quarter of the row of Dinv
-  T xs[NRC];
+  T xs = T(0);
 #pragma unroll
-  for (int c = 0; c < NRC; ++c) {
-    T sum = T(0);
-#pragma unroll
-    for (int i = 0; i < SEG; ++i) sum += Dinv[r][q * SEG + i] * accs[q * SEG + i][c];
-    xs[c] = sum;
-  }
-#pragma unroll
-  for (int c = 0; c < NRC; ++c) {
-    xs[c] += __shfl_xor(xs[c], 1);
-    xs[c] += __shfl_xor(xs[c], 2);
-  }
+  for (int i = 0; i < SEG; ++i) xs += Dinv[r][q * SEG + i] * accs[q * SEG + i];
+  xs += __shfl_xor(xs, 1);
+  xs += __shfl_xor(xs, 2);
   if constexpr (kM) {
     // X_b -= M X_l once l's solution is here: every wave polls X_l's BS
     // words itself (lane l: words l, l + 64) and publishes its own rows, so
@@ -354,44 +317,51 @@ __global__ __launch_bounds__(4 * BS) void trsv_chain_kernel(int n, const T* __re
       for (int i = 0; i < SEG; ++i) m += mrow[i] * __uint_as_float(xwv[wv][q * SEG + i]);
       m += __shfl_xor(m, 1);
       m += __shfl_xor(m, 2);
-      xs[0] -= m;
+      xs -= m;
     }
   }
   // publish: the result, and its exchange words for the successors
   if (q == 0 && rvalid) {
-#pragma unroll
-    for (int c = 0; c < NRC; ++c)
-      if (c < nc) {
-        X[(int64_t)(c0 + c) * ldx + rb0 + r] = xs[c];
-        u64* dst = xw + ((size_t)(rb0 + r) * NRC + c) * NW;
-        if (NW == 2) {
-          const u64 bits = (u64)__double_as_longlong((double)xs[c]);
-          __hip_atomic_store(dst, ((u64)epoch << 32) | (unsigned)bits, __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_AGENT);
-          __hip_atomic_store(dst + 1, ((u64)epoch << 32) | (unsigned)(bits >> 32),
-                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        } else {
-          __hip_atomic_store(dst, ((u64)epoch << 32) | __float_as_uint((float)xs[c]),
-                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-      }
+    X[rb0 + r] = xs;
+    u64* dst = xw + (size_t)(rb0 + r) * NW;
+    if (NW == 2) {
+      const u64 bits = (u64)__double_as_longlong((double)xs);
+      __hip_atomic_store(dst, ((u64)epoch << 32) | (unsigned)bits, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(dst + 1, ((u64)epoch << 32) | (unsigned)(bits >> 32), __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    } else {
+      __hip_atomic_store(dst, ((u64)epoch << 32) | __float_as_uint((float)xs), __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    }
   }
 }
 
 }  // namespace
 
 // Solves op(T) X = X in place.  T is n x n; `rowmajor` selects its layout;
-// lower/unit select the triangle.  X is column-major n x nrhs.
+// lower/unit select the triangle.  X is column-major n x nrhs.  FP64 with two
+// or more columns goes to the matrix-product solver: it is ahead of chains of
+// four columns from the start (us, solver / chains: n = 64, 2 columns 36 / 82;
+// n = 1024, 2 columns 108 / 137 and 16 columns 109 / 160; n = 8192, 4 columns
+// 674 / 805 and 64 columns 822 / 4129).  FP32 columns (the refinement, which
+// solves one at a time) run one chain each.
 template <typename T>
 int trsv_device(eamd_handle* h, int n, const T* A, int64_t lda, bool rowmajor, bool lower,
                 bool unit, T* X, int64_t ldx, int nrhs) {
   if (n <= 0 || nrhs <= 0) return kOk;
+  PhaseScope ps(h, kPhTrsv, sizeof(T) * (0.5 * (double)n * n + 2.0 * (double)n * nrhs),
+                (double)n * n * nrhs);
+  if constexpr (sizeof(T) == 8) {
+    if (nrhs > 1) return trsm_blocked(h, n, A, lda, rowmajor, lower, unit, X, ldx, nrhs);
+  }
   static const int spin_limit = env_int("EAMD_TRSV_SPIN", kSpin);
-  constexpr int BS = 64, NRC = 4, kChains = 4;
+  // (128-row blocks measured slower: 7.4 vs 3.7 ms of FP32 solves per step at
+  // n = 16384)
+  constexpr int BS = 64;
   const int nblk = ceil_div(n, BS);
-  // error word | exchange words (kChains chains of NRC values per row, 32
-  // payload bits each)
-  const size_t nwords = (size_t)nblk * BS * NRC * kChains * (sizeof(T) / 4);
+  // error word | exchange words (32 payload bits each)
+  const size_t nwords = (size_t)nblk * BS * (sizeof(T) / 4);
   size_t need = 256 + sizeof(unsigned long long) * nwords;
   void* base = nullptr;
   bool fresh = h->ws.bytes[kWsStatus] < need;
@@ -403,41 +373,12 @@ int trsv_device(eamd_handle* h, int n, const T* A, int64_t lda, bool rowmajor, b
     EAMD_HIP(hipMemsetAsync(base, 0, h->ws.bytes[kWsStatus], h->stream));
     h->trsv_epoch = 0;
   }
-  PhaseScope ps(h, kPhTrsv, sizeof(T) * (0.5 * (double)n * n + 2.0 * (double)n * nrhs),
-                (double)n * n * nrhs);
-  if (nrhs == 1) {
-    // one right-hand side: one exchange word (per 32 payload bits) per row
-    // (128-row blocks measured slower: 7.4 vs 3.7 ms of solves per step at
-    // n = 16384)
-    constexpr int BS1 = 64;
-    const int nblk1 = ceil_div(n, BS1);
+  for (int c = 0; c < nrhs; ++c) {
     const unsigned epoch = (unsigned)++h->trsv_epoch;
-#define EAMD_TRSV1(RM, LO, UN)                                                                   \
-  hipLaunchKernelGGL((trsv_chain_kernel<T, RM, LO, UN, BS1, 1>), dim3(nblk1), dim3(4 * BS1), 0, \
-                     h->stream, n, A, lda, X, ldx, 0, 1, xw, epoch, err, 1, spin_limit)
-    if (rowmajor) {
-      if (lower) { if (unit) EAMD_TRSV1(true, true, true); else EAMD_TRSV1(true, true, false); }
-      else { if (unit) EAMD_TRSV1(true, false, true); else EAMD_TRSV1(true, false, false); }
-    } else {
-      if (lower) { if (unit) EAMD_TRSV1(false, true, true); else EAMD_TRSV1(false, true, false); }
-      else { if (unit) EAMD_TRSV1(false, false, true); else EAMD_TRSV1(false, false, false); }
-    }
-#undef EAMD_TRSV1
-    EAMD_HIP(hipGetLastError());
-    return kOk;
-  }
-  // several right-hand sides: chains of four columns, up to four chains in
-  // one launch.  A chain's step costs about linearly in its columns (n =
-  // 8192: 24 us per 64-row step with sixteen, 6.5 us with four), so chains
-  // run side by side instead of one wide chain (LLT solve with 16
-  // right-hand sides: 6.3 ms with one chain of sixteen, 6.7 ms with four
-  // chains of four one after the other).
-  for (int c0 = 0; c0 < nrhs;) {
-    const unsigned epoch = (unsigned)++h->trsv_epoch;
-    const int nch = std::min(kChains, ceil_div(nrhs - c0, NRC));
-#define EAMD_TRSV(RM, LO, UN)                                                                  \
-  hipLaunchKernelGGL((trsv_chain_kernel<T, RM, LO, UN, BS, NRC>), dim3(nblk * nch), dim3(256), \
-                     0, h->stream, n, A, lda, X, ldx, c0, nrhs, xw, epoch, err, nch, spin_limit)
+    T* x = X + (int64_t)c * ldx;
+#define EAMD_TRSV(RM, LO, UN)                                                                 \
+  hipLaunchKernelGGL((trsv_chain_kernel<T, RM, LO, UN, BS>), dim3(nblk), dim3(4 * BS), 0,     \
+                     h->stream, n, A, lda, x, xw, epoch, err, spin_limit)
     if (rowmajor) {
       if (lower) { if (unit) EAMD_TRSV(true, true, true); else EAMD_TRSV(true, true, false); }
       else { if (unit) EAMD_TRSV(true, false, true); else EAMD_TRSV(true, false, false); }
@@ -447,13 +388,16 @@ int trsv_device(eamd_handle* h, int n, const T* A, int64_t lda, bool rowmajor, b
     }
 #undef EAMD_TRSV
     EAMD_HIP(hipGetLastError());
-    c0 += nch * NRC;
   }
   return kOk;
 }
 
 int trsv_check_error(eamd_handle* h) {
-  if (!h->ws.ptr[kWsStatus]) return kOk;
+  if (!h->ws.ptr[kWsStatus]) {
+    // no chain has run: nothing to read, but the call still completes
+    EAMD_HIP(hipStreamSynchronize(h->stream));
+    return kOk;
+  }
   int e = 0;
   EAMD_HIP(hipMemcpyAsync(&e, h->ws.ptr[kWsStatus], sizeof(int), hipMemcpyDeviceToHost,
                           h->stream));
