@@ -16,6 +16,8 @@
 //                      "bottleneck" of LLT.h:357).
 // A failure is recorded on the device; later kernels of the same call see
 // it and return early, so no host synchronisation per block is needed.
+#include <type_traits>
+
 #include "common.h"
 #include "kernels.h"
 
@@ -374,26 +376,248 @@ __global__ void set_int_kernel(int* p, int v) {
 }  // namespace
 
 namespace {
-// LLT rank-one update, L L^T + sigma v v^T = L' L'^T, in place: one wave per
-// system, row i of the factor on lane i % 64 (up to 4 rows per lane, n <=
-// 256).  Restates internal::llt_rank_update_lower (LLT.h:231-299): for
-// sigma > 0 a Givens rotation per column (JacobiRotation::makeGivens for
-// reals, Jacobi.h:226-262, applied as x' = c x + s y, y' = -s x + c y,
-// Jacobi.h:315-330); otherwise the scalar downdate, stopping at the first
-// column whose new diagonal would not be positive.  Column j's rows are read
-// and written by their own lanes in step j only, and the diagonal element
-// (j, j) is read by all lanes before lane j % 64 writes it, so the steps
-// need no other synchronisation.  info: -1, the failing column, or -2 for a
-// size outside 0..256.
+// LLT rank-one update, L L^T + sigma v v^T = L' L'^T, in place.  Restates
+// internal::llt_rank_update_lower (LLT.h:231-299): for sigma > 0 a Givens
+// rotation per column (JacobiRotation::makeGivens for reals, Jacobi.h:226-262,
+// applied as x' = c x + s y, y' = -s x + c y, Jacobi.h:315-330); otherwise the
+// scalar downdate, stopping at the first column whose new diagonal would not
+// be positive.  Column j is read and written in step j only, so its values
+// can be requested any number of steps ahead.  info: -1, the failing column,
+// or -2 for a size outside 0..256.
+//
+// A step is a chain of two divisions and a square root followed by a few
+// products per row, so lanes that repeat it for the same factor are lost
+// issue slots (1M factors of n = 6..24, a launch: one wave per factor 3.70 ms,
+// eight lanes per factor 1.12 ms = 1.9 TB/s of lower triangles).  Spans of 32 consecutive factors whose largest size is at most
+// 32 take eight lanes per factor, eight factors in step on a wave
+// (llt_rank_update_small_kernel); the others take one wave per factor.  Both
+// kernels run over every span and each skips the other's.
 constexpr int kRankUpdMaxN = 256;
-__global__ __launch_bounds__(256) void llt_rank_update_kernel(
+constexpr int kRankSpan = 32;  // factors that choose their kernel together
+constexpr int kRankLanes = 8;  // lanes of a small factor: row i on lane i % 8, slot i / 8
+
+template <int B, int E, typename F>
+__device__ __forceinline__ void sfor(F&& f) {
+  if constexpr (B < E) {
+    f(std::integral_constant<int, B>{});
+    sfor<B + 1, E>(f);
+  }
+}
+
+// the value of lane N of each group of eight lanes (row_newbcast: lane N of a
+// row of sixteen to the banks of its first group, lane 8 + N to its second)
+template <int N>
+__device__ __forceinline__ int bcast8(int x) {
+  const int lo = __builtin_amdgcn_update_dpp(x, x, 0x150 + N, 0xf, 0x3, false);
+  return __builtin_amdgcn_update_dpp(lo, x, 0x150 + 8 + N, 0xf, 0xc, false);
+}
+template <int N>
+__device__ __forceinline__ double bcast8(double x) {
+  const long long b = __double_as_longlong(x);
+  return __longlong_as_double(((long long)bcast8<N>((int)(b >> 32)) << 32) |
+                              (unsigned)bcast8<N>((int)b));
+}
+
+// makeGivens(p, q) for reals without its branches (lanes of a wave hold
+// different factors); the same operations in the same order.
+__device__ __forceinline__ void make_givens(double p, double q, double& c, double& sn,
+                                            double& r) {
+  const bool big = fabs(p) > fabs(q);
+  const double num = big ? q : p, den = big ? p : q;
+  const double tt = num / den;
+  double u = sqrt(1.0 + tt * tt);
+  if (den < 0.0) u = -u;
+  const double iu = 1.0 / u;
+  const double s2 = -iu;
+  c = big ? iu : -tt * s2;
+  sn = big ? -tt * iu : s2;
+  r = den * u;
+  if (p == 0.0) {
+    c = 0.0;
+    sn = q < 0.0 ? 1.0 : -1.0;
+    r = fabs(q);
+  }
+  if (q == 0.0) {
+    c = p < 0.0 ? -1.0 : 1.0;
+    sn = 0.0;
+    r = fabs(p);
+  }
+}
+
+// Whether the span's factors all have at most 32 rows (wave-uniform).
+__device__ __forceinline__ bool rank_span_small(int64_t span0, int64_t count,
+                                                const int32_t* __restrict__ nv, int lane,
+                                                int& size) {
+  size = lane < kRankSpan && span0 + lane < count ? nv[span0 + lane] : 0;
+  return __ballot(size > 8 * kRankLanes / 2) == 0;
+}
+
+// The updates (UP: sigma > 0) or downdates of eight factors, eight lanes
+// each; n = 0 for a lane whose factor is not of that kind.  Columns go in
+// groups of eight: a group's rows are loaded together, taken through eight
+// steps in registers and stored together.  Row i is on lane i % 8 of its
+// factor; slot r of group g holds rows 8 (g + r) .. 8 (g + r) + 7, so the
+// diagonal rows of a group are always slot 0.  Rows past n hold zeros and rows
+// above the current column values that are not stored, so a step needs no row
+// masks.  Returns the failing column or -1.
+// UPPER: the factor is stored transposed.
+template <bool UP, bool UPPER>
+__device__ __forceinline__ int rank_update_small(int n, double* __restrict__ L,
+                                                 const double* __restrict__ v, double sigma) {
+  constexpr int K = 4;
+  const int sl = threadIdx.x % kRankLanes;
+  int nmax = n;
+#pragma unroll
+  for (int off = 8; off < 64; off <<= 1) nmax = max(nmax, __shfl_xor(nmax, off));
+  nmax = __builtin_amdgcn_readfirstlane(nmax);
+  double t[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int i = sl + 8 * k;
+    t[k] = i < n ? v[i] : 0.0;
+  }
+  if (UP) {
+    const double ss = sqrt(sigma);
+#pragma unroll
+    for (int k = 0; k < K; ++k) t[k] = ss * t[k];
+  }
+  int ret = -1;
+  double beta = 1.0;
+#pragma unroll 1
+  for (int j0 = 0; j0 < nmax; j0 += 8) {
+    double x[K][8];
+    // element (j0 + sl, j0); one direction of the group is contiguous, the
+    // other goes by a running pointer (64 addresses at once cost a wave of
+    // occupancy)
+    double* Lg = L + j0 * (n + 1) + (UPPER ? sl * n : sl);
+    auto each = [&](auto&& f) {
+      double* p = Lg;
+      if constexpr (UPPER) {
+#pragma unroll
+        for (int r = 0; r < K; ++r) {
+          if (j0 + 8 * r >= nmax) break;
+          const bool in = j0 + 8 * r + sl < n;
+#pragma unroll
+          for (int q = 0; q < 8; ++q) f(in && (r > 0 || sl >= q), p + q, x[r][q]);
+          p += 8 * n;
+          asm volatile("" : "+v"(p));
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+#pragma unroll
+          for (int r = 0; r < K; ++r)
+            f(j0 + 8 * r + sl < n && (r > 0 || sl >= q), p + 8 * r, x[r][q]);
+          p += n;
+          asm volatile("" : "+v"(p));
+        }
+      }
+    };
+    each([](bool in, double* p, double& y) { y = in ? *p : 0.0; });
+    sfor<0, 8>([&](auto qc) {
+      constexpr int q = decltype(qc)::value;
+      if (j0 + q >= nmax) return;
+      const double tj = bcast8<q>(t[0]), p = bcast8<q>(x[0][q]);
+      double nd;  // the new diagonal
+      if constexpr (UP) {
+        double c, sn;
+        make_givens(p, -tj, c, sn, nd);
+        // the identity rotation leaves the column and the work vector as they
+        // are (Jacobi.h:460-461), also where they hold non-finite values
+        const bool ident = c == 1.0 && sn == 0.0;
+        const bool any = __ballot(ident) != 0;
+#pragma unroll
+        for (int r = 0; r < K; ++r) {
+          if (j0 + 8 * r >= nmax) break;
+          const double xi = x[r][q], y = t[r];
+          double out = c * xi + sn * y, tn = -sn * xi + c * y;
+          if (any) {
+            out = ident ? xi : out;
+            tn = ident ? y : tn;
+          }
+          x[r][q] = out;
+          t[r] = tn;
+        }
+        if (sl == q) x[0][q] = nd;
+      } else {
+        const double Ljj = p, dj = Ljj * Ljj, wj = tj;
+        const double swj2 = sigma * wj * wj, gamma = dj * beta + swj2;
+        const double xx = dj + swj2 / beta;
+        if (ret < 0 && j0 + q < n && xx <= 0.0) ret = j0 + q;
+        nd = sqrt(xx);
+        beta += swj2 / dj;
+        const double wl = wj / Ljj, a = nd / Ljj, b = nd * sigma * wj / gamma;
+        // a zero gamma leaves the rows; a failed factor changes no more
+        const bool stay = gamma == 0.0 || ret >= 0;
+        const bool any = __ballot(stay) != 0;
+#pragma unroll
+        for (int r = 0; r < K; ++r) {
+          if (j0 + 8 * r >= nmax) break;
+          const double xi = x[r][q], tn = t[r] - wl * xi;
+          double out = a * xi + b * tn;
+          if (any) out = stay ? xi : out;
+          x[r][q] = out;
+          t[r] = tn;
+        }
+        if (sl == q) x[0][q] = ret < 0 ? nd : p;
+      }
+    });
+    each([](bool in, double* p, double& y) {
+      if (in) *p = y;
+    });
+#pragma unroll
+    for (int r = 0; r + 1 < K; ++r) t[r] = t[r + 1];
+  }
+  return ret;
+}
+
+// One span per workgroup, eight factors per wave.
+__global__ __launch_bounds__(256, 3) void llt_rank_update_small_kernel(
     int64_t count, const int64_t* __restrict__ offL, const int32_t* __restrict__ nv,
     double* __restrict__ Lall, const int64_t* __restrict__ offv, const double* __restrict__ V,
     const double* __restrict__ sigmas, int upper, int32_t* __restrict__ info) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int64_t span0 = (int64_t)blockIdx.x * kRankSpan;
+  int size;
+  if (!rank_span_small(span0, count, nv, lane, size)) return;
+  const int sub = 8 * wave + lane / kRankLanes;  // this lane's factor in the span
+  const int64_t s = span0 + sub;
+  const bool act = s < count;
+  const int nr = __shfl(size, sub), n = max(nr, 0);
+  double* L = Lall + (n > 0 ? offL[s] : 0);
+  const double* v = V + (n > 0 ? offv[s] : 0);
+  const double sigma = act && sigmas ? sigmas[s] : 1.0;
+  const bool up = sigma > 0.0;
+  int ret = -1;
+  if (__ballot(up && n > 0) != 0) {
+    const int m = up ? n : 0;
+    if (upper) (void)rank_update_small<true, true>(m, L, v, sigma);
+    else (void)rank_update_small<true, false>(m, L, v, sigma);
+  }
+  if (__ballot(!up && n > 0) != 0) {
+    const int m = up ? 0 : n;
+    const int f = upper ? rank_update_small<false, true>(m, L, v, sigma)
+                        : rank_update_small<false, false>(m, L, v, sigma);
+    ret = up ? -1 : f;
+  }
+  if (act && lane % kRankLanes == 0) info[s] = nr < 0 ? -2 : ret;
+}
+
+// One wave per factor, row i on lane i % 64 (up to 4 rows per lane), for the
+// spans with a size above 32.  `spans` != 0: a workgroup walks a whole span, a
+// wave eight factors of it (many factors: skipping a span is one workgroup);
+// otherwise a workgroup has four factors.  Column j's rows are read and
+// written by their own lanes in step j only, and the diagonal element (j, j)
+// is read by all lanes before lane j % 64 writes it, so the steps need no
+// other synchronisation.
+__device__ void rank_update_wave(int64_t s, const int64_t* __restrict__ offL,
+                                 const int32_t* __restrict__ nv, double* __restrict__ Lall,
+                                 const int64_t* __restrict__ offv, const double* __restrict__ V,
+                                 const double* __restrict__ sigmas, int upper,
+                                 int32_t* __restrict__ info) {
   constexpr int K = kRankUpdMaxN / 64;
   const int lane = threadIdx.x & 63;
-  const int64_t s = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 6;
-  if (s >= count) return;  // whole waves
   const int n = nv[s];
   if (n < 0 || n > kRankUpdMaxN) {
     if (lane == 0) info[s] = -2;
@@ -486,19 +710,41 @@ __global__ __launch_bounds__(256) void llt_rank_update_kernel(
   }
   if (lane == 0) info[s] = ret;
 }
+
+__global__ __launch_bounds__(256) void llt_rank_update_kernel(
+    int64_t count, int spans, const int64_t* __restrict__ offL, const int32_t* __restrict__ nv,
+    double* __restrict__ Lall, const int64_t* __restrict__ offv, const double* __restrict__ V,
+    const double* __restrict__ sigmas, int upper, int32_t* __restrict__ info) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int64_t span0 = spans ? (int64_t)blockIdx.x * kRankSpan
+                              : (int64_t)(blockIdx.x / 8) * kRankSpan;
+  int size;
+  if (rank_span_small(span0, count, nv, lane, size)) return;
+  const int first = spans ? 8 * wave : 4 * (int)(blockIdx.x % 8) + wave, many = spans ? 8 : 1;
+  for (int q = 0; q < many; ++q) {
+    const int64_t s = span0 + first + q;
+    if (s < count) rank_update_wave(s, offL, nv, Lall, offv, V, sigmas, upper, info);
+  }
+}
 }  // namespace
 
 int llt_rank_update_batched(eamd_handle* h, int64_t count, const int64_t* offL, const int32_t* n,
                             double* L, const int64_t* offv, const double* v, const double* sigma,
                             int upper, int32_t* info) {
   if (count <= 0) return kOk;
-  const int64_t blocks = (count + 3) / 4;  // four waves (systems) per workgroup
-  if (blocks > INT32_MAX) {
+  const int64_t nspan = (count + kRankSpan - 1) / kRankSpan;
+  if (8 * nspan > INT32_MAX) {
     set_error("rank update: %lld systems exceed one launch", (long long)count);
     return kErrUnsupported;
   }
-  hipLaunchKernelGGL(llt_rank_update_kernel, dim3((unsigned)blocks), dim3(256), 0, h->stream,
+  hipLaunchKernelGGL(llt_rank_update_small_kernel, dim3((unsigned)nspan), dim3(256), 0, h->stream,
                      count, offL, n, L, offv, v, sigma, upper, info);
+  // with 2048 spans a wave for every eight factors still fills the chip
+  const int spans = nspan >= 2048 ? 1 : 0;
+  hipLaunchKernelGGL(llt_rank_update_kernel, dim3((unsigned)(spans ? nspan : 8 * nspan)),
+                     dim3(256), 0, h->stream, count, spans, offL, n, L, offv, v, sigma, upper,
+                     info);
   EAMD_HIP(hipGetLastError());
   return kOk;
 }
