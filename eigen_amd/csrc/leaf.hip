@@ -7,9 +7,9 @@
 // column by the pivot and the rank-1 update of the leaf.
 //
 // MI355X mapping.  Every thread keeps one row of the leaf (32 values) in
-// registers, so the rank-1 update is register FMAs; a workgroup holds
-// BLOCK rows (512 in FP64, 1024 in FP32) and at most 32 workgroups cover a
-// 16384-row panel.  With several workgroups, each column costs ONE memory
+// registers, so the rank-1 update is register FMAs; a workgroup holds 1024
+// rows (512 in FP64 when that is the whole leaf), and at most 32 (FP64: 16)
+// workgroups take part.  With several workgroups, each column costs ONE memory
 // round trip: every workgroup publishes its candidate (value, row) together
 // with the whole candidate row, and the owner of row j publishes row j, all
 // as 8-byte words carrying 32 bits of payload and the column's epoch (an
@@ -36,11 +36,6 @@ struct Words {
   static constexpr int n = sizeof(T) / 4;  // 32-bit payload words per value
 };
 
-template <typename T>
-struct LeafBlock {
-  static constexpr int v = sizeof(T) == 8 ? 512 : 1024;  // rows per workgroup
-};
-
 __device__ __forceinline__ void put_word(u64* p, unsigned payload, unsigned epoch) {
   __hip_atomic_store(p, ((u64)epoch << 32) | payload, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -62,11 +57,6 @@ __device__ __forceinline__ void put_value(u64* p, T v, unsigned epoch) {
 // in scratch memory).
 __device__ __forceinline__ float mask_sel(unsigned m, float x, float y) {
   return __uint_as_float((__float_as_uint(x) & m) | (__float_as_uint(y) & ~m));
-}
-__device__ __forceinline__ double mask_sel(unsigned m, double x, double y) {
-  const unsigned long long mm = ((unsigned long long)m << 32) | m;
-  return __longlong_as_double((long long)(((unsigned long long)__double_as_longlong(x) & mm) |
-                                          ((unsigned long long)__double_as_longlong(y) & ~mm)));
 }
 
 template <typename T>
@@ -162,6 +152,20 @@ __device__ __forceinline__ int readlane_i(int x, int lane) {
 }
 __device__ __forceinline__ float readlane_f(float x, int lane) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
+}
+
+// Maximum of a 32-bit key over the 64 lanes of a wave: xor-1 and xor-2
+// within quads, half-row and row mirrors within each 16-lane row, then the
+// row maxima are carried into lane 63 (row_bcast:15 into rows 1 and 3,
+// row_bcast:31 into rows 2 and 3).
+__device__ __forceinline__ unsigned wave_max_u32(unsigned k) {
+  k = max(k, (unsigned)__builtin_amdgcn_mov_dpp((int)k, 0xB1, 0xf, 0xf, false));
+  k = max(k, (unsigned)__builtin_amdgcn_mov_dpp((int)k, 0x4E, 0xf, 0xf, false));
+  k = max(k, (unsigned)__builtin_amdgcn_mov_dpp((int)k, 0x141, 0xf, 0xf, false));
+  k = max(k, (unsigned)__builtin_amdgcn_mov_dpp((int)k, 0x140, 0xf, 0xf, false));
+  k = max(k, (unsigned)__builtin_amdgcn_update_dpp((int)k, (int)k, 0x142, 0xa, 0xf, false));
+  k = max(k, (unsigned)__builtin_amdgcn_update_dpp((int)k, (int)k, 0x143, 0xc, 0xf, false));
+  return (unsigned)readlane_i((int)k, 63);
 }
 
 // The leaf-level permutation of a leaf's row interchanges, in registers (one
@@ -560,21 +564,382 @@ __global__ __launch_bounds__(BLOCK) void leaf_lu_kernel(
 }
 
 
+// ---------------------------------------------------------------------------
+// The FP64 leaf.  Same outputs and pivots as leaf_lu_kernel; what differs is
+// what a column costs (a 512-row leaf 82 -> 34 us, 1024 rows 133 -> 57 us,
+// 16384 rows 172 -> 112 us).  A thread holds one row (R = 1); up to 512 rows
+// take 512 threads and up to 1024 rows 1024, without an exchange, and 16384
+// rows sixteen such workgroups.  (Two rows on each of half the threads: 59 us
+// for 1024 rows.)  Rows never move: an interchange
+// relabels two positions, and each row is stored at its final position at the
+// end, so row j needs no publishing and nothing is selected by register masks.
+// The pivot search reduces the high words of |a| by DPP maxima and looks at
+// the low words and positions only on a tie.  The pivot row is read from LDS
+// once, one element per lane (lane c of every row of sixteen holds slots c and
+// 16 + c), and the rank-1 update takes it by the FMA's own lane broadcast
+// (v_fmac_f64 with row_newbcast): sixteen broadcast reads per wave and column
+// were a thousand LDS cycles.  Per column: one barrier after the waves'
+// candidates, then with one workgroup the pivot row through LDS and a second
+// barrier, with several the exchange (the candidate's wave publishes, all
+// poll, second barrier).
+constexpr int kLeaf64MaxG = 16;  // 16384 rows
+
+typedef double v2du __attribute__((ext_vector_type(2), aligned(8)));
+typedef double v2d __attribute__((ext_vector_type(2)));
+
+// a[C + q] += (lane (C + q) % 16 of each row of sixteen of u) * l for q = Q0
+// .. 7.  The wait states cover a VALU write of u just before (a DPP operand
+// needs two); they cost as much as an FMA, so one wait serves eight.
+template <int C, int Q0>
+__device__ __forceinline__ void fmac_bcast8(double (&a)[LW], double u, double l) {
+#define EAMD_FM(I, N) "v_fmac_f64_dpp %" #I ", %8, %9 row_newbcast:%" #N " row_mask:0xf bank_mask:0xf\n\t"
+  constexpr int N0 = C & 15;
+  if constexpr (Q0 == 0) {
+    asm volatile("s_nop 1\n\t" EAMD_FM(0, 10) EAMD_FM(1, 11) EAMD_FM(2, 12) EAMD_FM(3, 13)
+                     EAMD_FM(4, 14) EAMD_FM(5, 15) EAMD_FM(6, 16) EAMD_FM(7, 17)
+                 : "+v"(a[C]), "+v"(a[C + 1]), "+v"(a[C + 2]), "+v"(a[C + 3]), "+v"(a[C + 4]),
+                   "+v"(a[C + 5]), "+v"(a[C + 6]), "+v"(a[C + 7])
+                 : "v"(u), "v"(l), "n"(N0), "n"(N0 + 1), "n"(N0 + 2), "n"(N0 + 3), "n"(N0 + 4),
+                   "n"(N0 + 5), "n"(N0 + 6), "n"(N0 + 7));
+  } else {
+    // the current group's later columns: two at a time
+#define EAMD_F2(Q)                                                                              \
+  if constexpr (Q >= Q0)                                                                        \
+    asm volatile("s_nop 1\n\tv_fmac_f64_dpp %0, %2, %3 row_newbcast:%4 row_mask:0xf bank_mask:0xf\n\t" \
+                 "v_fmac_f64_dpp %1, %2, %3 row_newbcast:%5 row_mask:0xf bank_mask:0xf"        \
+                 : "+v"(a[C + Q]), "+v"(a[C + Q + 1])                                           \
+                 : "v"(u), "v"(l), "n"(N0 + Q), "n"(N0 + Q + 1));                               \
+  else if constexpr (Q + 1 >= Q0)                                                               \
+    asm volatile("s_nop 1\n\tv_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" \
+                 : "+v"(a[C + Q + 1])                                                           \
+                 : "v"(u), "v"(l), "n"(N0 + Q + 1));
+    EAMD_F2(0) EAMD_F2(2) EAMD_F2(4) EAMD_F2(6)
+#undef EAMD_F2
+  }
+#undef EAMD_FM
+}
+
+// Maximum over the lanes of each row of sixteen (all of them get it).
+__device__ __forceinline__ unsigned row_max_u32(unsigned k) {
+  k = max(k, (unsigned)__builtin_amdgcn_mov_dpp((int)k, 0xB1, 0xf, 0xf, false));
+  k = max(k, (unsigned)__builtin_amdgcn_mov_dpp((int)k, 0x4E, 0xf, 0xf, false));
+  k = max(k, (unsigned)__builtin_amdgcn_mov_dpp((int)k, 0x141, 0xf, 0xf, false));
+  return max(k, (unsigned)__builtin_amdgcn_mov_dpp((int)k, 0x140, 0xf, 0xf, false));
+}
+
+// Of the candidates (hi, lo, pos) on lanes 0..15 (repeated in every row of
+// sixteen; hi 0: none), the lane with the largest (hi, lo), lowest pos.
+__device__ __forceinline__ int row_best(unsigned hi, unsigned lo, unsigned pos) {
+  const unsigned mh = row_max_u32(hi);
+  unsigned b = (unsigned)__ballot(hi == mh) & 0xffffu;
+  if (__builtin_expect(__popc(b) != 1, 0)) {
+    const unsigned ml = row_max_u32(hi == mh ? lo : 0u);
+    const bool c = hi == mh && lo == ml;
+    const unsigned mp = row_max_u32(c ? ~pos : 0u);
+    b = (unsigned)__ballot(c && ~pos == mp) & 0xffffu;
+  }
+  return __builtin_amdgcn_readfirstlane(__ffs((int)b) - 1);
+}
+
+template <int NT, int R>
+__global__ __launch_bounds__(NT) void leaf64_kernel(
+    double* __restrict__ P, int64_t ldp, int m, int w, int G, int* __restrict__ piv,
+    int* __restrict__ lperm_n, int* __restrict__ lpos, int* __restrict__ lsrc,
+    int* __restrict__ pperm_n, int* __restrict__ ppos, int* __restrict__ psrc, int row0, int pnb,
+    int* __restrict__ zero_col, u64* __restrict__ xbuf, int* __restrict__ err,
+    unsigned epoch_base, int piv_offset, int* __restrict__ fz_global, int spin_limit) {
+  __builtin_amdgcn_s_setprio(3);  // on the critical path (see tsl_kernel)
+  constexpr int NWAVE = NT / 64;
+  constexpr int SW = slot_words<double>();  // [0] hi, [1] lo, [2] position, [3] unused, row
+  constexpr int STAGE = kLeaf64MaxG * SW, KMAX = (STAGE + NT - 1) / NT;
+  __shared__ uint4 s_key[2][NWAVE];           // each wave's candidate
+  __shared__ __align__(16) double s_row[LW];  // the workgroup's candidate row
+  __shared__ __align__(16) unsigned stage[STAGE];
+  __shared__ int s_abort;
+  __shared__ int s_piv[LW];
+  __shared__ __align__(16) int s_pp[256 + 4];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = blockIdx.x;
+
+  // slot r of a thread is row (g R + r) NT + tid, and pos its position (rows
+  // past m: none)
+  double v[R][LW];
+  int pos[R];
+  const double* src[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    pos[r] = (g * R + r) * NT + tid;
+    src[r] = P + (int64_t)min(pos[r], m - 1) * ldp;
+    if (pos[r] >= m) pos[r] = -1;
+  }
+  if (w == LW) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int c = 0; c < LW; c += 2) {
+        const v2du t = *reinterpret_cast<const v2du*>(src[r] + c);
+        v[r][c] = t.x;
+        v[r][c + 1] = t.y;
+      }
+  } else {
+#pragma unroll
+    for (int c = 0; c < LW; ++c) {
+      const int cc = min(c, w - 1);
+      const double on = c < w ? 1.0 : 0.0;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const double t = src[r][cc];
+        v[r][c] = on != 0.0 ? t : 0.0;
+      }
+    }
+  }
+  if (tid == 0) s_abort = 0;
+  __syncthreads();
+
+  int first_zero = -1;
+  // column j of group j / 8 is register slot jj (see rotate8); slots [live,
+  // 32) hold columns finished in earlier groups
+  auto column = [&](auto jjc, int j, int live) __attribute__((always_inline)) -> bool {
+    constexpr int jj = decltype(jjc)::value;
+    const int par = j & 1;
+    // ---- the wave's candidate: the largest |a| over rows at positions >= j by
+    // its high word (plus one: zero means none)
+    unsigned hi[R], lo[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const u64 b = (u64)__double_as_longlong(v[r][jj]);
+      hi[r] = pos[r] >= j ? ((unsigned)(b >> 32) & 0x7fffffffu) + 1u : 0u;
+      lo[r] = (unsigned)b;
+    }
+    unsigned mh = wave_max_u32(max(hi[0], hi[R - 1]));
+    if (__builtin_expect(mh > 0x7ff00000u, 0)) {
+      // infinities or NaNs: a NaN counts at position j only, as an infinity
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if (v[r][jj] != v[r][jj]) {
+          hi[r] = pos[r] == j ? 0x7ff00001u : 0u;
+          lo[r] = 0u;
+        }
+      mh = wave_max_u32(max(hi[0], hi[R - 1]));
+    }
+    u64 b0 = __ballot(hi[0] == mh), b1 = R == 2 ? __ballot(hi[R - 1] == mh) : 0ull;
+    if (__builtin_expect(__popcll(b0) + __popcll(b1) != 1 && mh != 0u, 0)) {
+      // equal high words: the low words, then the lowest position
+      const unsigned ml = wave_max_u32(max(hi[0] == mh ? lo[0] : 0u, hi[R - 1] == mh ? lo[R - 1] : 0u));
+      const bool c0 = hi[0] == mh && lo[0] == ml, c1 = hi[R - 1] == mh && lo[R - 1] == ml;
+      const unsigned mp = wave_max_u32(max(c0 ? ~(unsigned)pos[0] : 0u,
+                                           c1 ? ~(unsigned)pos[R - 1] : 0u));
+      b0 = __ballot(c0 && ~(unsigned)pos[0] == mp);
+      b1 = R == 2 ? __ballot(c1 && ~(unsigned)pos[R - 1] == mp) : 0ull;
+    }
+    const bool first = b0 != 0ull;
+    const int wl = __ffsll((long long)(first ? b0 : b1)) - 1;
+    if (lane == wl)
+      s_key[par][wave] = make_uint4(mh, first ? lo[0] : lo[R - 1],
+                                    (unsigned)(first ? pos[0] : pos[R - 1]),
+                                    (unsigned)lane + (first ? 0u : 64u));
+    __syncthreads();
+    // ---- the workgroup's candidate, found by every wave
+    const uint4 e = s_key[par][lane & (NWAVE - 1)];
+    // (with eight waves lanes 8..15 repeat their entries; without any candidate
+    // one of them may be named)
+    const int bw = row_best((lane & 15) < NWAVE ? e.x : 0u, e.y, e.z) & (NWAVE - 1);
+    int p = readlane_i((int)e.z, bw);
+    unsigned bhi = (unsigned)readlane_i((int)e.x, bw);
+    double u0, u1;
+    if (wave == bw) {
+      // its lane stores its row's live slots
+      const int code = readlane_i((int)e.w, bw);
+#define EAMD_PUT8(R_, C_)                                            \
+  _Pragma("unroll") for (int c = C_; c < C_ + 8; c += 2)              \
+    *reinterpret_cast<v2d*>(&s_row[c]) = v2d{v[R_][c], v[R_][c + 1]};
+#define EAMD_PUT(R_)                        \
+  if (lane == (code & 63)) {                \
+    EAMD_PUT8(R_, 0)                        \
+    if (live > 8) { EAMD_PUT8(R_, 8) }      \
+    if (live > 16) { EAMD_PUT8(R_, 16) }    \
+    if (live > 24) { EAMD_PUT8(R_, 24) }    \
+  }                                         \
+  /* (keeps the two copies apart: merged, the row would be indexed) */ \
+  asm volatile("; slot " #R_ ::: "memory");
+      if (R == 1 || code < 64) {
+        EAMD_PUT(0)
+      } else {
+        EAMD_PUT(R - 1)
+      }
+#undef EAMD_PUT
+#undef EAMD_PUT8
+    }
+    if (G == 1) {
+      __syncthreads();
+      u0 = s_row[lane & 15];
+      u1 = s_row[16 + (lane & 15)];
+    } else {
+      const unsigned epoch = epoch_base + (unsigned)j + 1u;
+      u64* base = xbuf + (size_t)par * G * SW;
+      if (wave == bw) {
+        // publish: the row a word per lane, and the header
+        asm volatile("" ::: "memory");  // a wave's LDS accesses execute in order
+        u64* slot = base + (size_t)g * SW;
+        const unsigned rw = reinterpret_cast<const unsigned*>(s_row)[lane];
+        const unsigned hw = lane == 0 ? bhi
+                            : lane == 1 ? (unsigned)readlane_i((int)e.y, bw)
+                            : lane == 2 ? (unsigned)p
+                                        : 0u;
+        if (lane < 4) put_word(slot + lane, hw, epoch);
+        put_word(slot + 4 + lane, rw, epoch);
+      }
+      // one parallel poll of every slot: each thread requests its words
+      // together, then only the missing ones again
+      const int total = G * SW;
+      bool done[KMAX];
+#pragma unroll
+      for (int k = 0; k < KMAX; ++k) done[k] = tid + k * NT >= total;
+      int bad = 0;
+      for (int spins = 0;; ++spins) {
+        u64 wv[KMAX];
+#pragma unroll
+        for (int k = 0; k < KMAX; ++k)
+          if (!done[k])
+            wv[k] = __hip_atomic_load(base + tid + k * NT, __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_AGENT);
+        bool all = true;
+#pragma unroll
+        for (int k = 0; k < KMAX; ++k)
+          if (!done[k]) {
+            if ((unsigned)(wv[k] >> 32) == epoch) {
+              stage[tid + k * NT] = (unsigned)wv[k];
+              done[k] = true;
+            } else {
+              all = false;
+            }
+          }
+        if (all) break;
+        // the limit every poll, another workgroup's give-up every 256th
+        if (spins >= spin_limit ||
+            ((spins & 255) == 255 &&
+             __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+          bad = 1;
+          break;
+        }
+      }
+      if (bad) s_abort = 1;
+      __syncthreads();
+      if (__builtin_expect(s_abort, 0)) {
+        if (tid == 0) __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return false;
+      }
+      const unsigned* hh = &stage[min(lane & 15, G - 1) * SW];
+      const unsigned sh = (lane & 15) < G ? hh[0] : 0u, slo = hh[1], sp = hh[2];
+      const int ws = row_best(sh, slo, sp);
+      p = readlane_i((int)sp, ws);
+      const double* ur = reinterpret_cast<const double*>(&stage[ws * SW + 4]);
+      u0 = ur[lane & 15];
+      u1 = ur[16 + (lane & 15)];
+    }
+    if (g == 0 && tid == 0) s_piv[j] = p;
+    // ---- positions j and p change places; the pivot row is at j and done.
+    // Then scale and rank-1 update of the rows below j (l = 0 leaves a row)
+    const double pv = readlane_d(u0, jj);
+    if (pv == 0.0 && first_zero < 0) first_zero = j;
+    double nl[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      pos[r] = pos[r] == p ? j : (pos[r] == j ? p : pos[r]);
+      const bool act = pos[r] > j && pv != 0.0;
+      const double q = v[r][jj] / pv;
+      nl[r] = act ? -q : 0.0;
+      v[r][jj] = act ? q : v[r][jj];
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if constexpr (jj < 7) fmac_bcast8<0, jj + 1>(v[r], u0, nl[r]);
+    if (live > 8) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) fmac_bcast8<8, 0>(v[r], u0, nl[r]);
+      if (live > 16) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) fmac_bcast8<16, 0>(v[r], u1, nl[r]);
+        if (live > 24) {
+#pragma unroll
+          for (int r = 0; r < R; ++r) fmac_bcast8<24, 0>(v[r], u1, nl[r]);
+        }
+      }
+    }
+    return true;
+  };
+  const int ngroups = (w + 7) / 8;
+  bool ok = true;
+#pragma unroll 1
+  for (int g8 = 0; g8 < ngroups && ok; ++g8) {
+    const int live = LW - 8 * g8, j0 = 8 * g8;
+#define EAMD_COL(JJ) \
+    if (ok && j0 + JJ < w) ok = column(std::integral_constant<int, JJ>{}, j0 + JJ, live);
+    EAMD_COL(0) EAMD_COL(1) EAMD_COL(2) EAMD_COL(3) EAMD_COL(4) EAMD_COL(5) EAMD_COL(6)
+    EAMD_COL(7)
+#undef EAMD_COL
+#pragma unroll
+    for (int r = 0; r < R; ++r) rotate8(v[r]);
+  }
+#pragma unroll 1
+  for (int q = ngroups; q < 4; ++q)
+#pragma unroll
+    for (int r = 0; r < R; ++r) rotate8(v[r]);
+  if (s_abort) {
+    // gave up: empty lists, as leaf_lu_kernel
+    if (g == 0 && tid == 0) {
+      *lperm_n = 0;
+      *pperm_n = 0;
+      *zero_col = -1;
+    }
+    return;
+  }
+  __syncthreads();
+  if (g == 0 && wave == 0) {
+    int tpos, trow, tsrc, ln;
+    leaf_lists<false>(lane < w ? s_piv[lane] : 0, w, row0, pnb, lane, piv, piv_offset, lperm_n,
+                      lpos, lsrc, pperm_n, ppos, psrc, s_pp, tpos, trow, tsrc, ln);
+  }
+  // every row at its final position (every workgroup has read its rows before
+  // any passes the exchange of a column)
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (pos[r] < 0) continue;
+    double* dst = P + (int64_t)pos[r] * ldp;
+    if (w == LW) {
+#pragma unroll
+      for (int c = 0; c < LW; c += 2)
+        *reinterpret_cast<v2du*>(dst + c) = v2du{v[r][c], v[r][c + 1]};
+    } else {
+#pragma unroll
+      for (int c = 0; c < LW; ++c)
+        if (c < w) dst[c] = v[r][c];
+    }
+  }
+  if (g == 0 && tid == 0) {
+    *zero_col = first_zero;
+    if (fz_global && first_zero >= 0 && *fz_global < 0) *fz_global = first_zero + piv_offset;
+  }
+}
+
 // Launches one leaf over rows [0, m) of the sub-panel at P (row-major, ldp),
 // columns [0, w), w <= 32.
 template <typename T>
 int leaf_lu(eamd_handle* h, T* P, int64_t ldp, int m, int w, int* piv, int* lperm_n, int* lpos,
             int* lsrc, int* pperm_n, int* ppos, int* psrc, int row0, int pnb, int* zero_col,
             int piv_offset, int* fz_global) {
-  constexpr int BLOCK = LeafBlock<T>::v;
   if (w > LW || pnb > 256) {
     set_error("leaf width %d / panel width %d unsupported", w, pnb);
     return kErrUnsupported;
   }
-  const int G = ceil_div(m, BLOCK);
-  if (G > kMaxG) {
-    set_error("panel of %d rows exceeds the leaf exchange (%d workgroups of %d rows)", m, kMaxG,
-              BLOCK);
+  constexpr bool k64 = sizeof(T) == 8;
+  constexpr int BLOCK = 1024;
+  const int rows = k64 && m <= 512 ? 512 : BLOCK;
+  const int G = ceil_div(m, rows), max_g = k64 ? kLeaf64MaxG : kMaxG;
+  if (G > max_g) {
+    set_error("panel of %d rows exceeds the leaf exchange (%d workgroups of %d rows)", m, max_g,
+              rows);
     return kErrUnsupported;
   }
   const int SW = slot_words<T>();
@@ -592,10 +957,18 @@ int leaf_lu(eamd_handle* h, T* P, int64_t ldp, int m, int w, int* piv, int* lper
   // polls an exchange may take before the leaf gives up (the call then
   // reports a time-out); EAMD_LEAF_SPIN sets another limit
   static const int spin_limit = env_int("EAMD_LEAF_SPIN", kLeafSpin);
-  hipLaunchKernelGGL((leaf_lu_kernel<T, BLOCK>), dim3(G), dim3(BLOCK), 0, h->stream, P, ldp, m, w,
-                     G, piv, lperm_n, lpos, lsrc, pperm_n, ppos, psrc, row0, pnb, zero_col,
-                     reinterpret_cast<u64*>(b + 256), reinterpret_cast<int*>(b), epoch_base,
-                     piv_offset, fz_global, spin_limit);
+#define EAMD_LEAF(K, NT)                                                                      \
+  hipLaunchKernelGGL((K), dim3(G), dim3(NT), 0, h->stream, P, ldp, m, w, G, piv, lperm_n, lpos, \
+                     lsrc, pperm_n, ppos, psrc, row0, pnb, zero_col,                          \
+                     reinterpret_cast<u64*>(b + 256), reinterpret_cast<int*>(b), epoch_base,  \
+                     piv_offset, fz_global, spin_limit)
+  if constexpr (k64) {
+    if (m > 512) EAMD_LEAF((leaf64_kernel<1024, 1>), 1024);
+    else EAMD_LEAF((leaf64_kernel<512, 1>), 512);
+  } else {
+    EAMD_LEAF((leaf_lu_kernel<T, BLOCK>), BLOCK);
+  }
+#undef EAMD_LEAF
   EAMD_HIP(hipGetLastError());
   return kOk;
 }
@@ -627,20 +1000,6 @@ constexpr int kTslR = 4;                 // rows per lane
 constexpr int kTslBlock = 64 * kTslR;    // rows (candidates) per wave
 constexpr int kTslFan = kTslBlock / LW;  // candidate groups merged per wave
 constexpr int kMoveCols = 96;            // panel columns moved per pass in the final round
-
-// Maximum of a 32-bit key over the 64 lanes of a wave: xor-1 and xor-2
-// within quads, half-row and row mirrors within each 16-lane row, then the
-// row maxima are carried into lane 63 (row_bcast:15 into rows 1 and 3,
-// row_bcast:31 into rows 2 and 3).
-__device__ __forceinline__ unsigned wave_max_u32(unsigned k) {
-  k = max(k, (unsigned)__builtin_amdgcn_mov_dpp((int)k, 0xB1, 0xf, 0xf, false));
-  k = max(k, (unsigned)__builtin_amdgcn_mov_dpp((int)k, 0x4E, 0xf, 0xf, false));
-  k = max(k, (unsigned)__builtin_amdgcn_mov_dpp((int)k, 0x141, 0xf, 0xf, false));
-  k = max(k, (unsigned)__builtin_amdgcn_mov_dpp((int)k, 0x140, 0xf, 0xf, false));
-  k = max(k, (unsigned)__builtin_amdgcn_update_dpp((int)k, (int)k, 0x142, 0xa, 0xf, false));
-  k = max(k, (unsigned)__builtin_amdgcn_update_dpp((int)k, (int)k, 0x143, 0xc, 0xf, false));
-  return (unsigned)readlane_i((int)k, 63);
-}
 
 // Lane `me` stores its register row v[rs] (rs wave-uniform) to LDS as eight
 // 16-byte words: a scalar branch over the slot, then the one lane's stores.
