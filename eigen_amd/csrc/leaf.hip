@@ -169,41 +169,38 @@ __device__ __forceinline__ unsigned wave_max_u32(unsigned k) {
 }
 
 // The leaf-level permutation of a leaf's row interchanges, in registers (one
-// wave): entry k (lane k < ln) is leaf row tpos, which receives the content
-// of entry tsrc and so holds original row trow (rows 0..w-1 are entries
-// 0..w-1, rows swapped in from below are appended).  FROM_SEL: lane c < w
-// holds x = the original row selected for row c, and x returns the
-// transposition of column c (the row swapped with row c); otherwise x is
-// that transposition.
-template <bool FROM_SEL>
-__device__ __forceinline__ void leaf_perm(int& x, int w, int lane, int& tpos, int& trow,
-                                          int& tsrc, int& ln) {
-  tpos = lane < w ? lane : -1;
-  trow = tpos;
-  tsrc = lane;
-  int nent = w, pivv = 0;
-  for (int c = 0; c < w; ++c) {
-    const int p = readlane_i(x, c);
-    const u64 hit = __ballot((FROM_SEL ? trow : tpos) == p);
+// wave): entry k (lane k < n) is leaf row pos, which receives the content of
+// entry src and so holds original row row (rows 0..w-1 are entries 0..w-1,
+// rows swapped in from below are appended).
+struct LeafPerm {
+  int pos, row, src, n;
+  __device__ __forceinline__ void start(int w, int lane) {
+    pos = lane < w ? lane : -1;
+    row = pos;
+    src = lane;
+    n = w;
+  }
+  // Column c's interchange with entry k, the entry of position p (FROM_SEL: of
+  // original row p); an untouched row p (>= w) sits at position p and becomes
+  // a new entry (*fresh).
+  template <bool FROM_SEL>
+  __device__ __forceinline__ int step(int c, int p, int lane, bool* fresh = nullptr) {
+    const u64 hit = __ballot((FROM_SEL ? row : pos) == p);
     int k;
     if (hit) {
       k = __ffsll((long long)hit) - 1;
-    } else {  // an untouched row p (>= w) sits at position p
-      k = nent++;
-      if (lane == k) { tpos = p; trow = p; tsrc = k; }
+    } else {
+      k = n++;
+      if (lane == k) { pos = p; row = p; src = k; }
     }
-    if (FROM_SEL) {
-      const int pk = readlane_i(tpos, k);
-      if (lane == c) pivv = pk;
-    }
-    const int rc = readlane_i(trow, c), rk = readlane_i(trow, k);
-    const int sc = readlane_i(tsrc, c), sk = readlane_i(tsrc, k);
-    if (lane == c) { trow = rk; tsrc = sk; }
-    if (lane == k) { trow = rc; tsrc = sc; }
+    if (fresh) *fresh = !hit;
+    const int rc = readlane_i(row, c), rk = readlane_i(row, k);
+    const int sc = readlane_i(src, c), sk = readlane_i(src, k);
+    if (lane == c) { row = rk; src = sk; }
+    if (lane == k) { row = rc; src = sc; }
+    return k;
   }
-  if (FROM_SEL) x = pivv;
-  ln = nent;
-}
+};
 
 // Composes a leaf's list (lane k < ln: leaf row tpos receives the content of
 // entry tsrc) into the panel-level list ppos/psrc/pperm_n (the leaf starts at
@@ -214,8 +211,7 @@ __device__ __forceinline__ void leaf_perm(int& x, int w, int lane, int& tpos, in
 // The panel's first leaf (row0 == 0) starts the list as the identity.  One
 // wave; s_pp is LDS scratch of at least pnb + 4 ints.
 __device__ void panel_compose(int tpos, int tsrc, int ln, int row0, int pnb, int lane,
-                              int* pperm_n, int* ppos, int* psrc, int* s_pp, const int* s_ps,
-                              int pn0_pre) {
+                              int* pperm_n, int* ppos, int* psrc, int* s_pp) {
   const bool first = row0 == 0;
   if (first) {
     for (int e = lane; e < pnb; e += 64) {
@@ -225,12 +221,8 @@ __device__ void panel_compose(int tpos, int tsrc, int ln, int row0, int pnb, int
     // complete before the touched slots are stored over them
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
-  // pn0_pre >= 0: the incoming list was prefetched (count pn0_pre, appended
-  // rows in s_pp padded with -1 to a multiple of 4, sources in s_ps)
-  const bool pre = pn0_pre >= 0;
-  const int pn0 = first ? pnb : (pre ? pn0_pre : *pperm_n), na = pn0 - pnb, na4 = (na + 3) & ~3;
-  if (!pre)
-    for (int e = lane; e < na4; e += 64) s_pp[e] = e < na ? ppos[pnb + e] : -1;
+  const int pn0 = first ? pnb : *pperm_n, na = pn0 - pnb, na4 = (na + 3) & ~3;
+  for (int e = lane; e < na4; e += 64) s_pp[e] = e < na ? ppos[pnb + e] : -1;
   asm volatile("" ::: "memory");  // LDS accesses of one wave execute in order
   const bool mine = lane < ln;
   const int prow = row0 + tpos;
@@ -251,7 +243,7 @@ __device__ void panel_compose(int tpos, int tsrc, int ln, int row0, int pnb, int
   const u64 nb = __ballot(need);
   if (need) slot = pn0 + __popcll(nb & ((1ull << lane) - 1ull));
   int old = slot;
-  if (mine && !need && !first) old = pre ? s_ps[slot] : psrc[slot];
+  if (mine && !need && !first) old = psrc[slot];
   const int src_old = __shfl(old, tsrc);
   if (mine) {
     psrc[slot] = src_old;
@@ -260,22 +252,22 @@ __device__ void panel_compose(int tpos, int tsrc, int ln, int row0, int pnb, int
   if (lane == 0) *pperm_n = pn0 + __popcll(nb);
 }
 
-// All lists of a leaf from its interchanges (one wave): piv[] (plus
-// piv_offset), the leaf-level list lperm_n/lpos/lsrc and the panel-level one.
-// FROM_SEL as for leaf_perm; tpos/trow/tsrc return the leaf list's entries.
-template <bool FROM_SEL>
+// All lists of a leaf from its interchanges (one wave; lane c < w: x = the row
+// swapped with row c): piv[] (plus piv_offset), the leaf-level list
+// lperm_n/lpos/lsrc and the panel-level one.
 __device__ void leaf_lists(int x, int w, int row0, int pnb, int lane, int* piv, int piv_offset,
                            int* lperm_n, int* lpos, int* lsrc, int* pperm_n, int* ppos,
-                           int* psrc, int* s_pp, int& tpos, int& trow, int& tsrc, int& ln,
-                           const int* s_ps = nullptr, int pn0_pre = -1) {
-  leaf_perm<FROM_SEL>(x, w, lane, tpos, trow, tsrc, ln);
+                           int* psrc, int* s_pp) {
+  LeafPerm lp;
+  lp.start(w, lane);
+  for (int c = 0; c < w; ++c) lp.step<false>(c, readlane_i(x, c), lane);
   if (lane < w) piv[lane] = x + piv_offset;
-  if (lane < ln) {
-    lpos[lane] = tpos;
-    lsrc[lane] = tsrc;
+  if (lane < lp.n) {
+    lpos[lane] = lp.pos;
+    lsrc[lane] = lp.src;
   }
-  if (lane == 0) *lperm_n = ln;
-  panel_compose(tpos, tsrc, ln, row0, pnb, lane, pperm_n, ppos, psrc, s_pp, s_ps, pn0_pre);
+  if (lane == 0) *lperm_n = lp.n;
+  panel_compose(lp.pos, lp.src, lp.n, row0, pnb, lane, pperm_n, ppos, psrc, s_pp);
 }
 
 }  // namespace
@@ -547,9 +539,8 @@ __global__ __launch_bounds__(BLOCK) void leaf_lu_kernel(
   // ---- bookkeeping (workgroup 0, wave 0): the leaf-level and panel-level
   // permutation lists, replaying the interchanges in column order
   if (g == 0 && wave == 0) {
-    int tpos, trow, tsrc, ln;
-    leaf_lists<false>(lane < w ? s_piv[lane] : 0, w, row0, pnb, lane, piv, piv_offset, lperm_n,
-                      lpos, lsrc, pperm_n, ppos, psrc, s_pp, tpos, trow, tsrc, ln);
+    leaf_lists(lane < w ? s_piv[lane] : 0, w, row0, pnb, lane, piv, piv_offset, lperm_n, lpos,
+               lsrc, pperm_n, ppos, psrc, s_pp);
   }
   if (valid) {
     T* dst = P + (int64_t)i * ldp;
@@ -897,9 +888,8 @@ __global__ __launch_bounds__(NT) void leaf64_kernel(
   }
   __syncthreads();
   if (g == 0 && wave == 0) {
-    int tpos, trow, tsrc, ln;
-    leaf_lists<false>(lane < w ? s_piv[lane] : 0, w, row0, pnb, lane, piv, piv_offset, lperm_n,
-                      lpos, lsrc, pperm_n, ppos, psrc, s_pp, tpos, trow, tsrc, ln);
+    leaf_lists(lane < w ? s_piv[lane] : 0, w, row0, pnb, lane, piv, piv_offset, lperm_n, lpos,
+               lsrc, pperm_n, ppos, psrc, s_pp);
   }
   // every row at its final position (every workgroup has read its rows before
   // any passes the exchange of a column)
@@ -980,57 +970,119 @@ int leaf_lu(eamd_handle* h, T* P, int64_t ldp, int m, int w, int* piv, int* lper
 // by the backward error after refinement rather than by Eigen's pivot
 // sequence.  A leaf of m rows costs a few short launches instead of one
 // exchange round trip per column:
-//   1. one wave per 256 rows (two waves per 512 rows when more than 32
-//      groups would follow) runs partial pivoting on them, in registers, and
-//      records the rows it picked (up to 32 candidates);
-//   2. while more than 32 candidate groups remain, one wave per 8 groups runs
-//      partial pivoting on the original values of their candidates and keeps
-//      32 of them;
-//   3. one workgroup does the same over the last groups (one wave for at
-//      most 8, four waves for at most 32, each column's pivot the largest of
-//      the waves' maxima): the rows it picks, in order, are the leaf's pivots
-//      and its first 32 rows after elimination are the factored top block
-//      L11\U11, written in place; its first wave also saves the original rows
-//      0..w-1, derives the transpositions, replays them into the permutation
-//      lists and lists where the displaced rows go;
+//   1. a workgroup per 256, 512 or 1024 rows (see leaf_lu_tournament) runs
+//      partial pivoting on them, in registers, and records the rows it picked
+//      (up to 32 candidates);
+//   2. while more groups remain than one workgroup's rows hold, a workgroup
+//      per 16 groups (8 with the wide rounds off) runs partial pivoting on the
+//      original values of their candidates and keeps 32 of them;
+//   3. one workgroup does the same over the last groups: the rows it picks, in
+//      order, are the leaf's pivots, and each is a row of the factored top
+//      block L11\U11 as it is picked, written in place; a wave without rows
+//      keeps the books: it saves the original rows 0..w-1, derives the
+//      transpositions, replays them into the permutation lists and lists where
+//      the displaced rows go;
 //   4. every other row is solved against U11 (l = a U11^-1) in parallel.
 namespace {
 
-constexpr int kTslR = 4;                 // rows per lane
-constexpr int kTslBlock = 64 * kTslR;    // rows (candidates) per wave
-constexpr int kTslFan = kTslBlock / LW;  // candidate groups merged per wave
-constexpr int kMoveCols = 96;            // panel columns moved per pass in the final round
+// Shape of a round's workgroup over CAP rows (or candidates): a row per thread
+// up to 512 (a wave per SIMD, then two), two rows per thread for 1024.  The
+// final round's bookkeeping wave comes on top.  What bounds it: the columns
+// follow each other, and a column is some 60 instructions of search, exchange
+// and scaling per wave beside its FMAs, so a lone wave of each SIMD with four
+// rows per lane issued one every six cycles and waited on LDS in between
+// (1024 rows in four waves: 2000 cycles a column; 512 in two: 1650; 256 in
+// one: 1350).  The registers stay within what one of the trailing update's
+// workgroups gives back when it ends (272 per SIMD): a round that needed the
+// room of two would wait until the update drains.
+template <int CAP>
+struct Tsl {
+  static constexpr int R = CAP == 1024 ? 2 : 1;  // rows per thread
+  static constexpr int NW = CAP / 64 / R;        // waves with rows
+  static constexpr int KB = CAP == 256 ? 9 : (CAP == 512 ? 10 : 11);
+  static_assert((1 << KB) == 2 * CAP, "slot code width");
+};
 
-// Lane `me` stores its register row v[rs] (rs wave-uniform) to LDS as eight
-// 16-byte words: a scalar branch over the slot, then the one lane's stores.
-__device__ __forceinline__ void put_row(float* dst, const float (&v)[kTslR][LW], int rs,
-                                        bool me) {
-#define EAMD_PUT(R_)                                                                   \
-  if (rs == R_) {                                                                      \
-    if (me) {                                                                          \
-      _Pragma("unroll") for (int q = 0; q < LW / 4; ++q)                               \
-        reinterpret_cast<float4*>(dst)[q] =                                            \
-            make_float4(v[R_][4 * q], v[R_][4 * q + 1], v[R_][4 * q + 2], v[R_][4 * q + 3]); \
-    }                                                                                  \
-    asm volatile("; slot " #R_ ::: "memory");                                          \
+// a[C + q] += (lane (C + q) % 16 of each row of sixteen of u) * l for q = Q0
+// .. 7 (as fmac_bcast8, in FP32).
+template <int C, int Q0>
+__device__ __forceinline__ void fmac_bcast8f(float (&a)[LW], float u, float l) {
+  constexpr int N0 = C & 15;
+  static_assert(Q0 == 0 || C == 0, "part groups start the row");
+#define EAMD_F(I, U, L, N)                                                                \
+  "v_fmac_f32_dpp %" #I ", %" #U ", %" #L " row_newbcast:" #N " row_mask:0xf bank_mask:0xf\n\t"
+#define EAMD_FN(I, N)                                                                     \
+  "v_fmac_f32_dpp %" #I ", %8, %9 row_newbcast:%" #N " row_mask:0xf bank_mask:0xf\n\t"
+  if constexpr (Q0 == 0) {
+    asm volatile("s_nop 1\n\t" EAMD_FN(0, 10) EAMD_FN(1, 11) EAMD_FN(2, 12) EAMD_FN(3, 13)
+                     EAMD_FN(4, 14) EAMD_FN(5, 15) EAMD_FN(6, 16) EAMD_FN(7, 17)
+                 : "+v"(a[C]), "+v"(a[C + 1]), "+v"(a[C + 2]), "+v"(a[C + 3]), "+v"(a[C + 4]),
+                   "+v"(a[C + 5]), "+v"(a[C + 6]), "+v"(a[C + 7])
+                 : "v"(u), "v"(l), "n"(N0), "n"(N0 + 1), "n"(N0 + 2), "n"(N0 + 3), "n"(N0 + 4),
+                   "n"(N0 + 5), "n"(N0 + 6), "n"(N0 + 7));
+  } else if constexpr (Q0 == 1) {
+    asm volatile("s_nop 1\n\t" EAMD_F(0, 7, 8, 1) EAMD_F(1, 7, 8, 2) EAMD_F(2, 7, 8, 3)
+                     EAMD_F(3, 7, 8, 4) EAMD_F(4, 7, 8, 5) EAMD_F(5, 7, 8, 6) EAMD_F(6, 7, 8, 7)
+                 : "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]),
+                   "+v"(a[7])
+                 : "v"(u), "v"(l));
+  } else if constexpr (Q0 == 2) {
+    asm volatile("s_nop 1\n\t" EAMD_F(0, 6, 7, 2) EAMD_F(1, 6, 7, 3) EAMD_F(2, 6, 7, 4)
+                     EAMD_F(3, 6, 7, 5) EAMD_F(4, 6, 7, 6) EAMD_F(5, 6, 7, 7)
+                 : "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7])
+                 : "v"(u), "v"(l));
+  } else if constexpr (Q0 == 3) {
+    asm volatile("s_nop 1\n\t" EAMD_F(0, 5, 6, 3) EAMD_F(1, 5, 6, 4) EAMD_F(2, 5, 6, 5)
+                     EAMD_F(3, 5, 6, 6) EAMD_F(4, 5, 6, 7)
+                 : "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7])
+                 : "v"(u), "v"(l));
+  } else if constexpr (Q0 == 4) {
+    asm volatile("s_nop 1\n\t" EAMD_F(0, 4, 5, 4) EAMD_F(1, 4, 5, 5) EAMD_F(2, 4, 5, 6)
+                     EAMD_F(3, 4, 5, 7)
+                 : "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7])
+                 : "v"(u), "v"(l));
+  } else if constexpr (Q0 == 5) {
+    asm volatile("s_nop 1\n\t" EAMD_F(0, 3, 4, 5) EAMD_F(1, 3, 4, 6) EAMD_F(2, 3, 4, 7)
+                 : "+v"(a[5]), "+v"(a[6]), "+v"(a[7])
+                 : "v"(u), "v"(l));
+  } else if constexpr (Q0 == 6) {
+    asm volatile("s_nop 1\n\t" EAMD_F(0, 2, 3, 6) EAMD_F(1, 2, 3, 7)
+                 : "+v"(a[6]), "+v"(a[7])
+                 : "v"(u), "v"(l));
+  } else if constexpr (Q0 == 7) {
+    asm volatile("s_nop 1\n\t" EAMD_F(0, 1, 2, 7) : "+v"(a[7]) : "v"(u), "v"(l));
   }
-  EAMD_PUT(0) else EAMD_PUT(1) else EAMD_PUT(2) else EAMD_PUT(3)
-#undef EAMD_PUT
+#undef EAMD_FN
+#undef EAMD_F
 }
 
-// One wave per block of up to 256 candidate rows, 4 rows per lane, all in
-// registers.  MODE 0: local selection over rows blockIdx.x*256 + [0, 256),
-// candidates to cand.  MODE 2: merge of candidate groups [8 b, 8 b + 8) of
-// cand_in into group b of cand.  MODE 1: the final round over all G_in
-// (<= 8) groups.  With NW > 1 waves a workgroup covers NW such blocks (MODE
-// 0: NW*256 rows; MODE 1: up to 8*NW groups, wave q holding groups
-// [8q, 8q + 8)): every column's pivot is the maximum over the waves' own
-// maxima, exchanged through LDS under one barrier.
-template <int MODE, int NW>
-__global__ __launch_bounds__(64 * NW) void tsl_kernel(
-    float* __restrict__ P, int64_t ldp, int m, int w, const int* __restrict__ cand_in,
-    const int* __restrict__ cand_n_in, int G_in, int* __restrict__ cand,
-    int* __restrict__ cand_n, float* __restrict__ saved, int* __restrict__ moved,
+template <int C>
+__device__ __forceinline__ void fmac_bcast1f(float (&a)[LW], float u, float l) {
+  asm volatile("s_nop 1\n\tv_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+               : "+v"(a[C])
+               : "v"(u), "v"(l), "n"(C));
+}
+
+// The largest of NK (16 or 32) keys in LDS, on every lane.
+template <int NK>
+__device__ __forceinline__ unsigned keys_max(const unsigned* s_key, int lane) {
+  unsigned k = s_key[lane & 15];
+  if (NK == 32) k = max(k, s_key[16 + (lane & 15)]);
+  return row_max_u32(k);
+}
+
+// MODE 0: local selection over rows blockIdx.x * CAP + [0, CAP), candidates
+// to cand.  MODE 2: merge of the n_in candidates' CAP / 32 groups from
+// blockIdx.x * CAP / 32 on into group blockIdx.x of cand.  MODE 1: the final
+// round over all n_in candidates (at most CAP / 32 groups).  Every candidate
+// group is full (w candidates) but the last.  A column's pivot is the maximum
+// over the waves' own maxima, exchanged through LDS; the pivot row is read from
+// LDS once, an element per lane, and the update takes it by the FMA's lane
+// broadcast (see leaf64_kernel).
+template <int MODE, int CAP>
+__global__ __launch_bounds__(64 * (Tsl<CAP>::NW + (MODE == 1))) void tsl_kernel(
+    float* __restrict__ P, int64_t ldp, int m, int w, const int* __restrict__ cand_in, int n_in,
+    int* __restrict__ cand, float* __restrict__ saved, int* __restrict__ moved,
     int* __restrict__ piv, int* __restrict__ lperm_n, int* __restrict__ lpos,
     int* __restrict__ lsrc, int* __restrict__ pperm_n, int* __restrict__ ppos,
     int* __restrict__ psrc, int row0, int pnb, int* __restrict__ zero_col, int piv_offset,
@@ -1038,347 +1090,314 @@ __global__ __launch_bounds__(64 * NW) void tsl_kernel(
   // the panel is the factorization's critical path while the trailing
   // update's waves share its SIMDs: its waves take issue priority
   __builtin_amdgcn_s_setprio(3);
-  constexpr int R = kTslR;
-  static_assert(MODE != 2 || NW == 1, "merge rounds run one wave per workgroup");
-  // slot ids in the key's low KB bits: 2^KB = 2 * NW * 256 keeps every
-  // id's code (2^KB - 1 - slot) nonzero
-  constexpr int KB = NW == 1 ? 9 : (NW == 2 ? 10 : 11);
+  constexpr int R = Tsl<CAP>::R, NW = Tsl<CAP>::NW, KB = Tsl<CAP>::KB;
+  constexpr int NT = 64 * (NW + (MODE == 1)), WROWS = 64 * R;
   constexpr unsigned kSlotMask = (1u << KB) - 1u;
-  static_assert((1 << KB) == 2 * NW * kTslBlock, "slot code width");
-  __shared__ int s_sel[LW];
-  __shared__ __align__(16) int s_pp[256 + 4];
-  __shared__ __align__(16) float s_u[LW];  // the pivot row of the current column
-  __shared__ __align__(16) float s_rows[NW > 1 ? 2 : 1][NW][LW];  // each wave's best row
-  __shared__ unsigned s_key[NW > 1 ? 2 : 1][NW];                  // and its key
-  const int lane = threadIdx.x & 63;
-  const int wave = NW > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;
-  // MODE 1: the incoming panel list's count (the lists themselves are
-  // prefetched below, while the columns are eliminated)
-  int pn0_pre = -1;
-  if (MODE == 1) pn0_pre = row0 == 0 ? pnb : *pperm_n;
-  // MODE 1: the original rows 0..w-1 (saved before the top block overwrites
-  // them), loaded first and stored last
-  float sv[LW * LW / 64];
-  if (MODE == 1 && wave == 0) {
+  __shared__ unsigned s_key[4 * NW];         // each sixteen lanes' largest key
+  __shared__ __align__(16) float s_row[LW];  // the pivot row
+  __shared__ __align__(16) float s_in[NW][64 * LW];  // rows on their way to their lanes
+  __shared__ int s_orig[MODE == 1 ? CAP : 1];        // each slot's row
+  // the bookkeeping wave's lists, for the final moves
+  __shared__ int s_pos[64], s_src[64], s_ps[MODE == 1 ? 512 : 1], s_n;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int s0 = MODE == 1 ? 0 : blockIdx.x * (MODE == 0 ? CAP : CAP / LW * w);
+  const int nrows = min(MODE == 0 ? CAP : CAP / LW * w, (MODE == 0 ? m : n_in) - s0);
+  const int steps = min(w, nrows);
+  if (MODE != 1 || wave < NW) {
+    // slot q = WROWS wave + 64 r + lane
+    int orig[R];
+    unsigned em[R], kq[R];
+    int st[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int q = wave * WROWS + r * 64 + lane;
+      const bool valid = q < nrows;
+      // (groups of w candidates, LW apart)
+      const int e = s0 + q;
+      orig[r] = !valid ? 0
+                       : (MODE == 0 ? e : cand_in[w == LW ? e : (e / w) * LW + e % w]);
+      if (MODE == 1) s_orig[q] = orig[r];
+      em[r] = valid ? ~0u : 0u;
+      kq[r] = kSlotMask - (unsigned)q;
+      st[r] = -1;
+    }
+    // An empty slot loads row 0 and a leaf narrower than 32 repeats its last
+    // column: such values are never keyed, selected or stored.
+    float v[R][LW];
+    if (w == LW && ((uintptr_t)P & 15) == 0 && (ldp & 3) == 0) {
+      // eight lanes per row, so that a load instruction asks for eight whole
+      // 128-byte lines (a row per lane: 64 lines, eight times over), then
+      // through LDS to the rows' lanes.  Word c of row i lies at c ^ (i % 8):
+      // consecutive lanes' 16-byte reads fall on different banks.
+      v4f t[R][8];
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const int row = __shfl(orig[r], 8 * k + (lane >> 3));
+          t[r][k] = reinterpret_cast<const v4f*>(P + (int64_t)row * ldp)[lane & 7];
+        }
+      v4f* buf = reinterpret_cast<v4f*>(s_in[wave]);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          buf[(8 * k + (lane >> 3)) * 8 + ((lane & 7) ^ (lane >> 3))] = t[r][k];
+        asm volatile("" ::: "memory");  // a wave's LDS accesses execute in order
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+          const v4f x = buf[lane * 8 + (c ^ (lane & 7))];
+          v[r][4 * c] = x.x;
+          v[r][4 * c + 1] = x.y;
+          v[r][4 * c + 2] = x.z;
+          v[r][4 * c + 3] = x.w;
+        }
+        asm volatile("" ::: "memory");
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const float* src = P + (int64_t)orig[r] * ldp;
+#pragma unroll
+        for (int c = 0; c < LW; ++c) v[r][c] = src[w == LW ? c : min(c, w - 1)];
+      }
+    }
+    // every row read before the final round's first top row is stored
+    if (MODE == 1) {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int c = 0; c < LW; ++c) asm volatile("" : "+v"(v[r][c])::"memory");
+    }
+    // Rows never move between lanes.  A slot holds a candidate row while em[r]
+    // is all ones (valid and not yet selected); st[r] is the step that
+    // selected it.  The pivot key of slot q is |a| with its KB low mantissa
+    // bits replaced by 2^KB - 1 - q (zero for a slot that is out), so the
+    // maximum names its slot, exact ties go to the lowest slot (the first row
+    // in order for the local round) and scores within 2^(KB-23) relative count
+    // as ties, which keeps every multiplier within 1 + 2^(KB-23).  Column j
+    // of group g8 is register slot jj (see rotate8); slots [live, 32) hold
+    // columns of earlier groups and are skipped by uniform branches on 8-slot
+    // chunks, so the update does exactly the triangle.  The multipliers use
+    // the reciprocal of the pivot.
+    // the wave's key of the column in slot c
+    auto post_key = [&](auto cc) __attribute__((always_inline)) {
+      constexpr int c = decltype(cc)::value;
+      unsigned key = 0;
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        key = max(key, ((__float_as_uint(v[r][c]) & (0x7fffffffu & ~kSlotMask)) | kq[r]) & em[r]);
+      key = row_max_u32(key);
+      if ((lane & 15) == 0) s_key[tid >> 4] = key;
+    };
+    // A column: the keys are out at the first barrier; the slot of the largest
+    // stores its row, out at the second; the next column's slot is
+    // updated first, so that its keys are searched and out while the rest of
+    // the update runs.  (With every wave storing its own best row instead, for
+    // one barrier less, the single-lane stores alone were 500 cycles with four
+    // waves and 1000 with eight.)  A valid unselected slot exists (j <
+    // steps), so the winner does.
+    auto column = [&](auto jjc, int j, int live) __attribute__((always_inline)) {
+      constexpr int jj = decltype(jjc)::value;
+      __syncthreads();
+      const unsigned code = keys_max<4 * NW>(s_key, lane) & kSlotMask;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const bool sel = kq[r] == code;
+        if (sel) {
+          float4* dst = reinterpret_cast<float4*>(s_row);
+#pragma unroll
+          for (int c = 0; c < LW / 4; ++c)
+            dst[c] = make_float4(v[r][4 * c], v[r][4 * c + 1], v[r][4 * c + 2], v[r][4 * c + 3]);
+          asm volatile("" ::: "memory");
+        }
+        em[r] = sel ? 0u : em[r];
+        st[r] = sel ? j : st[r];
+      }
+      __syncthreads();
+      const float u0 = s_row[lane & 15], u1 = s_row[16 + (lane & 15)];
+      const float pv = readlane_f(u0, jj);
+      const float rinv = pv != 0.f ? __builtin_amdgcn_rcpf(pv) : 0.f;
+      float nl[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const float l = v[r][jj] * rinv;
+        nl[r] = __uint_as_float((__float_as_uint(l) ^ 0x80000000u) & em[r]);
+        v[r][jj] = em[r] ? l : v[r][jj];
+      }
+      if (jj < 7) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) fmac_bcast1f<(jj + 1) % 8>(v[r], u0, nl[r]);
+        if (j + 1 < steps) post_key(std::integral_constant<int, (jj + 1) % 8>{});
+#pragma unroll
+        for (int r = 0; r < R; ++r) fmac_bcast8f<0, jj + 2>(v[r], u0, nl[r]);
+      }
+      if (live > 8)
+#pragma unroll
+        for (int r = 0; r < R; ++r) fmac_bcast8f<8, 0>(v[r], u0, nl[r]);
+      if (jj == 7 && j + 1 < steps) post_key(std::integral_constant<int, 8>{});
+      if (live > 16)
+#pragma unroll
+        for (int r = 0; r < R; ++r) fmac_bcast8f<16, 0>(v[r], u1, nl[r]);
+      if (live > 24)
+#pragma unroll
+        for (int r = 0; r < R; ++r) fmac_bcast8f<24, 0>(v[r], u1, nl[r]);
+    };
+    post_key(std::integral_constant<int, 0>{});
+#pragma unroll 1
+    for (int j0 = 0; j0 < steps; j0 += 8) {
+      const int live = LW - j0;
+#define EAMD_COL(JJ) \
+  if (j0 + JJ < steps) column(std::integral_constant<int, JJ>{}, j0 + JJ, live);
+      EAMD_COL(0) EAMD_COL(1) EAMD_COL(2) EAMD_COL(3) EAMD_COL(4) EAMD_COL(5) EAMD_COL(6)
+      EAMD_COL(7)
+#undef EAMD_COL
+#pragma unroll
+      for (int r = 0; r < R; ++r) rotate8(v[r]);
+    }
+    if (MODE != 1) {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if (st[r] >= 0) cand[blockIdx.x * LW + st[r]] = orig[r];
+    }
+  } else {
+    // ---- the bookkeeping wave of the final round.  The original rows 0..w-1,
+    // read before the top block overwrites them:
 #pragma unroll
     for (int k = 0; k < LW * LW / 64; ++k) {
       const int e = lane + 64 * k, r = e / LW, c = e % LW;
-      sv[k] = P[(int64_t)r * ldp + min(c, w - 1)];
+      const float x = P[(int64_t)r * ldp + min(c, w - 1)];
+      saved[e] = c < w ? x : 0.f;
     }
-  }
-  int orig[R];
-  bool valid[R];
-  int nrows;  // candidates of the workgroup
-  if (MODE == 0) {
-    const int wg0 = blockIdx.x * (NW * kTslBlock), base = wg0 + wave * kTslBlock;
-    nrows = min(NW * kTslBlock, m - wg0);
-    const int nw = min(kTslBlock, m - base);
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int q = r * 64 + lane;
-      valid[r] = q < nw;
-      orig[r] = valid[r] ? base + q : 0;
-    }
-  } else {
-    // the workgroup's group counts, one per lane, and their inclusive
-    // prefix sums; wave q's groups are [8q, 8q + 8) of the workgroup's
-    constexpr int NG = NW * kTslFan;
-    const int gb = MODE == 2 ? blockIdx.x * kTslFan : 0;
-    const int nga = max(0, min(NG, G_in - gb));
-    int inc = lane < nga ? cand_n_in[gb + lane] : 0;
-#pragma unroll
-    for (int d = 1; d < NG; d <<= 1) {
-      const int t = __shfl_up(inc, d);
-      if (lane >= d) inc += t;
-    }
-    nrows = readlane_i(inc, NG - 1);
-    const int wg = wave * kTslFan;
-    const int pre = wave > 0 ? readlane_i(inc, wg - 1) : 0;
-    int off[kTslFan + 1];  // wave-uniform offsets of the wave's groups
-    off[0] = 0;
-#pragma unroll
-    for (int g = 0; g < kTslFan; ++g) off[g + 1] = readlane_i(inc, wg + g) - pre;
-    const int nw = off[kTslFan];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int q = r * 64 + lane;
-      valid[r] = q < nw;
-      // group of slot q: the last g whose offset is <= q (empty groups
-      // share their successor's offset)
-      int gs = 0, o = 0;
-#pragma unroll
-      for (int g = 1; g < kTslFan; ++g) {
-        const bool ge = q >= off[g];
-        gs = ge ? g : gs;
-        o = ge ? off[g] : o;
-      }
-      orig[r] = valid[r] ? cand_in[(gb + wg + gs) * LW + q - o] : 0;
-    }
-  }
-  // An empty slot loads row 0 and a leaf narrower than 32 repeats its last
-  // column: such values are never keyed, selected or stored.
-  float v[R][LW];
-  if (w == LW && ((uintptr_t)P & 15) == 0 && (ldp & 3) == 0) {
-    // 16-byte loads: a quarter of the address work of word loads, which
-    // otherwise saturates the CU's address unit when several waves load
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const v4f* src = reinterpret_cast<const v4f*>(P + (int64_t)orig[r] * ldp);
-#pragma unroll
-      for (int q = 0; q < LW / 4; ++q) {
-        const v4f t = src[q];
-        v[r][4 * q] = t.x;
-        v[r][4 * q + 1] = t.y;
-        v[r][4 * q + 2] = t.z;
-        v[r][4 * q + 3] = t.w;
-      }
-    }
-  } else if (w == LW) {
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const float* src = P + (int64_t)orig[r] * ldp;
-#pragma unroll
-      for (int c = 0; c < LW; ++c) v[r][c] = src[c];
-    }
-  } else {
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const float* src = P + (int64_t)orig[r] * ldp;
-#pragma unroll
-      for (int c = 0; c < LW; ++c) v[r][c] = src[min(c, w - 1)];
-    }
-  }
-  int ppv[4], psv[8];
-  if (MODE == 1) {
-    const bool has = row0 != 0 && wave == 0;
+    // the incoming panel list (row0 == 0 starts it as the identity): lane l
+    // keeps the appended rows l, l + 64, ..., LDS the sources
+    const bool first = row0 == 0;
+    const int pn0 = first ? pnb : *pperm_n;
+    int app[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int e = 64 * q + lane;
-      ppv[q] = (has && e < pn0_pre - pnb) ? ppos[pnb + e] : -1;
+      app[q] = !first && e < pn0 - pnb ? ppos[pnb + e] : -1;
     }
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int e = 64 * q + lane;
-      psv[q] = (has && e < pn0_pre) ? psrc[e] : 0;
-    }
-  }
-  const int steps = min(w, nrows);
-  int first_zero = -1;
-  // Rows never move between lanes.  Slot q = 256 wave + 64 r + lane holds a
-  // candidate row while em[r] is all ones (valid and not yet selected);
-  // st[r] is the step that selected it.  The pivot key of slot q is |a| with
-  // its KB low mantissa bits replaced by 2^KB - 1 - q (km = em & 0x7fffffff
-  // with those bits clear, kq = em & (2^KB - 1 - q); zero for a slot that is
-  // out), so the maximum names its slot, exact ties go to the lowest slot
-  // (the first row in order for the local round) and scores within
-  // 2^(KB-23) relative count as ties, which keeps every multiplier within
-  // 1 + 2^(KB-23) (2^-14 for one wave, 2^-12 for four).  Column j of group g8 is register slot jj
-  // (see rotate8); slots [live, 32) hold columns of earlier groups and are
-  // skipped by uniform branches on 8-slot chunks, so the update does exactly
-  // the triangle.  The multipliers use the reciprocal of the pivot.
-  unsigned em[R], km[R], kq[R];
-  int st[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    em[r] = valid[r] ? ~0u : 0u;
-    km[r] = em[r] & (0x7fffffffu & ~kSlotMask);
-    kq[r] = em[r] & (kSlotMask - (unsigned)(wave * kTslBlock + r * 64 + lane));
-    st[r] = -1;
-  }
-  auto column = [&](auto jjc, int j, int live) __attribute__((always_inline)) {
-    constexpr int jj = decltype(jjc)::value;
-    unsigned kr[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) kr[r] = (__float_as_uint(v[r][jj]) & km[r]) | kq[r];
-    const unsigned key = max(max(kr[0], kr[1]), max(kr[2], kr[3]));
-    // a valid unselected slot exists (j < steps), so the winner does
-    const unsigned wkey = wave_max_u32(key);
-    const int ql = (int)(kSlotMask - (wkey & kSlotMask)) - wave * kTslBlock;
-    int rs = ql >> 6, wl = ql & 63;
-    bool me = lane == wl;
-    const float* ub = s_u;
-    if constexpr (NW == 1) {
-      // the pivot row: stored by its lane, read back by all (a wave's LDS
-      // accesses execute in order; the barriers keep the compiler from
-      // moving the reads above the store)
-      put_row(s_u, v, rs, me);
-      asm volatile("" ::: "memory");
-    } else {
-      // every wave stores its best row and key (a wave without candidates
-      // has key 0 and decodes a slot outside its 256, so stores nothing),
-      // then all take the largest key: its wave's row is the pivot row.
-      // Column parity double-buffers the exchange: the stores of column
-      // j + 2 follow the barrier of column j + 1, after every read of j.
-      const int par = j & 1;
-      put_row(s_rows[par][wave], v, rs, me);
-      if (lane == 0) s_key[par][wave] = wkey;
-      __syncthreads();
-      unsigned gkey = s_key[par][0];
-#pragma unroll
-      for (int q = 1; q < NW; ++q) gkey = max(gkey, s_key[par][q]);
-      const int gw = (int)(kSlotMask - (gkey & kSlotMask)) >> 8;
-      me = me && gw == wave;
-      ub = s_rows[par][gw];
-    }
-    float u[LW];
-#pragma unroll
-    for (int q = 0; q < LW / 4; ++q) {
-      const float4 t = reinterpret_cast<const float4*>(ub)[q];
-      u[4 * q] = t.x;
-      u[4 * q + 1] = t.y;
-      u[4 * q + 2] = t.z;
-      u[4 * q + 3] = t.w;
-    }
-    asm volatile("" ::: "memory");
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-      if (rs == r && me) {
-        em[r] = 0u;
-        km[r] = 0u;
-        kq[r] = 0u;
-        st[r] = j;
+    for (int e = lane; e < 2 * pnb; e += 64) {
+      s_ps[e] = !first && e < pn0 ? psrc[e] : e;
+      if (first && e < pnb) {
+        ppos[e] = e;
+        psrc[e] = e;
       }
-    const float pv = u[jj];
-    if (pv == 0.f && first_zero < 0) first_zero = j;
-    const float rinv = pv != 0.f ? __builtin_amdgcn_rcpf(pv) : 0.f;
-    float l[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const unsigned lb = __float_as_uint(v[r][jj] * rinv);
-      l[r] = __uint_as_float(lb & em[r]);
-      v[r][jj] = __uint_as_float((lb & em[r]) | (__float_as_uint(v[r][jj]) & ~em[r]));
     }
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-#pragma unroll
-      for (int c = jj + 1; c < 8; ++c) v[r][c] = fmaf(-l[r], u[c], v[r][c]);
-    if (live > 8) {
-#pragma unroll
-      for (int r = 0; r < R; ++r)
-#pragma unroll
-        for (int c = 8; c < 16; ++c) v[r][c] = fmaf(-l[r], u[c], v[r][c]);
-    }
-    if (live > 16) {
-#pragma unroll
-      for (int r = 0; r < R; ++r)
-#pragma unroll
-        for (int c = 16; c < 24; ++c) v[r][c] = fmaf(-l[r], u[c], v[r][c]);
-    }
-    if (live > 24) {
-#pragma unroll
-      for (int r = 0; r < R; ++r)
-#pragma unroll
-        for (int c = 24; c < 32; ++c) v[r][c] = fmaf(-l[r], u[c], v[r][c]);
-    }
-  };
-  const int ngroups = (steps + 7) / 8;
+    // complete before the lists and the top block are stored over
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    LeafPerm lp;
+    lp.start(w, lane);
+    // entry k's slot of the panel list (rows 0..pnb-1 are slots 0..pnb-1,
+    // rows below them are appended slots), found as the entry appears
+    int slot = row0 + lane, pn = pn0, first_zero = -1, my_piv = 0;
 #pragma unroll 1
-  for (int g8 = 0; g8 < ngroups; ++g8) {
-    const int live = LW - 8 * g8, j0 = 8 * g8;
-#define EAMD_COL(JJ) \
-    if (j0 + JJ < steps) column(std::integral_constant<int, JJ>{}, j0 + JJ, live);
-    EAMD_COL(0) EAMD_COL(1) EAMD_COL(2) EAMD_COL(3) EAMD_COL(4) EAMD_COL(5) EAMD_COL(6)
-    EAMD_COL(7)
-#undef EAMD_COL
+    for (int j = 0; j < steps; ++j) {
+      __syncthreads();
+      const unsigned code = keys_max<4 * NW>(s_key, lane) & kSlotMask;
+      const int p = __builtin_amdgcn_readfirstlane(s_orig[(int)(kSlotMask - code)]);
+      __syncthreads();
+      // the row picked is row j of the top block (slot s of group g8 holds
+      // column (s + 8 g8) % 32)
+      const float x = s_row[lane & (LW - 1)];
+      const int col = (lane + (j & ~7)) & (LW - 1);
+      if (lane < LW && col < w) P[(int64_t)j * ldp + col] = x;
+      if (readlane_f(x, j & 7) == 0.f && first_zero < 0) first_zero = j;
+      bool fresh;
+      const int k = lp.step<true>(j, p, lane, &fresh);
+      if (lane == j) my_piv = k;
+      if (fresh) {
+        const int prow = row0 + p;
+        int f = prow;
+        if (prow >= pnb) {
+          f = -1;
 #pragma unroll
-    for (int r = 0; r < R; ++r) rotate8(v[r]);
-  }
-  if (MODE != 1) {
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-      if (st[r] >= 0) cand[blockIdx.x * LW + st[r]] = orig[r];
-    if (threadIdx.x == 0) cand_n[blockIdx.x] = steps;
-    return;
+          for (int t = 0; t < 4; ++t) {
+            const u64 hit = __ballot(app[t] == prow);
+            if (hit) f = pnb + 64 * t + __ffsll((long long)hit) - 1;
+          }
+          if (f < 0) f = pn++;
+        }
+        if (lane == k) slot = f;
+      }
+    }
+    // ---- the leaf's lists: column c is swapped with entry k's position
+    const int ln = lp.n;
+    const int tp = __shfl(lp.pos, my_piv);
+    if (lane < w) piv[lane] = tp + piv_offset;
+    if (lane < ln) {
+      lpos[lane] = lp.pos;
+      lsrc[lane] = lp.src;
+    }
+    s_pos[lane] = lp.pos;
+    s_src[lane] = __shfl(lp.pos, lp.src);
+    // the panel's: a touched slot's new source is the old source of its
+    // entry's source slot, and an appended slot's old source is itself
+    const bool add = slot >= pn0;
+    int old = slot;
+    if (lane < ln && !add) old = s_ps[slot];
+    const int src_old = __shfl(old, lp.src);
+    if (lane < ln) {
+      psrc[slot] = src_old;
+      if (add) ppos[slot] = row0 + lp.pos;
+    }
+    // positions >= w now hold displaced original rows < w: list them
+    const bool mv = lane < ln && lp.pos >= w;
+    const u64 mb = __ballot(mv);
+    const int idx = __popcll(mb & ((1ull << lane) - 1ull));
+    if (mv) {
+      moved[1 + 2 * idx] = lp.pos;
+      moved[2 + 2 * idx] = lp.row;
+    }
+    if (lane == 0) {
+      s_n = ln;
+      moved[0] = __popcll(mb);
+      *lperm_n = ln;
+      *pperm_n = pn;
+      *zero_col = first_zero;
+      if (fz_global && first_zero >= 0 && *fz_global < 0) *fz_global = first_zero + piv_offset;
+    }
   }
   if constexpr (MODE == 1) {
-#pragma unroll 1
-  for (int q = ngroups; q < 4; ++q)
-#pragma unroll
-    for (int r = 0; r < R; ++r) rotate8(v[r]);
-  if (wave == 0) {
-#pragma unroll
-    for (int k = 0; k < LW * LW / 64; ++k) {
-      const int e = lane + 64 * k;
-      saved[e] = e % LW < w ? sv[k] : 0.f;
-    }
-  }
-  // ---- final round: the top block in place (rows 0..w-1) and the selection
-#pragma unroll
-  for (int r = 0; r < R; ++r)
-    if (st[r] >= 0) {
-      float* dst = P + (int64_t)st[r] * ldp;
-      if (w == LW && ((uintptr_t)P & 15) == 0 && (ldp & 3) == 0) {
-#pragma unroll
-        for (int q = 0; q < LW / 4; ++q)
-          reinterpret_cast<v4f*>(dst)[q] =
-              v4f{v[r][4 * q], v[r][4 * q + 1], v[r][4 * q + 2], v[r][4 * q + 3]};
-      } else {
-#pragma unroll
-        for (int c = 0; c < LW; ++c)
-          if (c < w) dst[c] = v[r][c];
-      }
-      s_sel[st[r]] = orig[r];
-    }
-  __syncthreads();
-  // the rest is one wave's (no barrier follows)
-  if (NW > 1 && wave != 0) return;
-  // ---- transpositions and permutation lists from the selection order
-  __shared__ int s_ps[512];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) s_pp[64 * q + lane] = ppv[q];
-#pragma unroll
-  for (int q = 0; q < 8; ++q) s_ps[64 * q + lane] = psv[q];
-  asm volatile("" ::: "memory");  // a wave's LDS accesses execute in order
-  int tpos, trow, tsrc, ln;
-  leaf_lists<true>(lane < w ? s_sel[lane] : 0, w, row0, pnb, lane, piv, piv_offset, lperm_n,
-                   lpos, lsrc, pperm_n, ppos, psrc, s_pp, tpos, trow, tsrc, ln, s_ps, pn0_pre);
-  // positions >= w now hold displaced original rows < w: list them
-  const bool mv = tpos >= w && lane < ln;
-  const u64 mb = __ballot(mv);
-  const int idx = __popcll(mb & ((1ull << lane) - 1ull));
-  if (mv) {
-    moved[1 + 2 * idx] = tpos;
-    moved[2 + 2 * idx] = trow;
-  }
-  if (lane == 0) moved[0] = __popcll(mb);
-  if (fuse) {
+    if (!fuse) return;
     // (w == 32) The leaf's interchanges on the other columns of the panel
-    // (row0 = j0 is the leaf's first panel column, pnb the panel width): the
-    // lane of each touched row moves its source row's values, 96 columns at
-    // a time (all loads of a chunk before its stores); the top rows' values
+    // (row0 = j0 is the leaf's first panel column, pnb the panel width), 96
+    // columns at a time, all loads before the stores; the top rows' values
     // right of the leaf go to xtop (LW x (pnb - j0 - LW)), from which the
-    // apply kernel solves U12.
-    const int srow = __shfl(tpos, tsrc);
-    const int j0 = row0, nc = pnb - LW, rest = pnb - j0 - LW;
+    // apply kernel solves U12.  16-byte words: the host fuses only panels
+    // whose rows start 16-byte aligned with pnb and ldp multiples of 4 (a word
+    // never straddles the leaf, whose columns start at a multiple of 32).
+    __syncthreads();
+    constexpr int CW = 24, NM = (64 * CW + NT - 1) / NT;  // words per pass, and per thread
+    const int ln = s_n, j0 = row0, nq = (pnb - LW) / 4, rest = pnb - j0 - LW;
     float* base = P - j0;  // panel column 0 of leaf row 0
-    // 16-byte words: the host fuses only panels whose rows start 16-byte
-    // aligned with pnb and ldp multiples of 4 (a word never straddles the
-    // leaf, whose columns start at a multiple of 32)
-    if (lane < ln) {
-      const v4f* sp = reinterpret_cast<const v4f*>(base + (int64_t)srow * ldp);
-      v4f* dp = reinterpret_cast<v4f*>(base + (int64_t)tpos * ldp);
-      v4f* xp = tpos < LW ? reinterpret_cast<v4f*>(xtop + tpos * rest) : nullptr;
-      const int nq = nc / 4;
-      for (int q0 = 0; q0 < nq; q0 += kMoveCols / 4) {
-        v4f x[kMoveCols / 4];
+    for (int q0 = 0; q0 < nq; q0 += CW) {
+      v4f x[NM];
 #pragma unroll
-        for (int t = 0; t < kMoveCols / 4; ++t) {
-          const int c = 4 * min(q0 + t, nq - 1);
-          x[t] = sp[(c < j0 ? c : c + LW) / 4];
-        }
+      for (int t = 0; t < NM; ++t) {
+        const int e = tid + NT * t, k = e / CW, c = 4 * (q0 + e % CW);
+        if (k < ln && c < 4 * nq)
+          x[t] = *reinterpret_cast<const v4f*>(base + (int64_t)s_src[k] * ldp +
+                                               (c < j0 ? c : c + LW));
+      }
+      // the loads of every wave are complete when its barrier is reached
 #pragma unroll
-        for (int t = 0; t < kMoveCols / 4; ++t) {
-          const int c = 4 * (q0 + t);
-          v4f* d = xp && c >= j0 ? xp + (c - j0) / 4 : dp + (c < j0 ? c : c + LW) / 4;
-          if (q0 + t < nq) *d = x[t];
+      for (int t = 0; t < NM; ++t) asm volatile("" : "+v"(x[t])::"memory");
+      __syncthreads();
+#pragma unroll
+      for (int t = 0; t < NM; ++t) {
+        const int e = tid + NT * t, k = e / CW, c = 4 * (q0 + e % CW);
+        if (k < ln && c < 4 * nq) {
+          const int tpos = s_pos[k];
+          float* d = tpos < LW && c >= j0 ? xtop + tpos * rest + (c - j0)
+                                          : base + (int64_t)tpos * ldp + (c < j0 ? c : c + LW);
+          *reinterpret_cast<v4f*>(d) = x[t];
         }
       }
     }
-  }
-  if (lane == 0) {
-    *zero_col = first_zero;
-    if (fz_global && first_zero >= 0 && *fz_global < 0) *fz_global = first_zero + piv_offset;
-  }
   }
 }
 
@@ -1459,12 +1478,16 @@ __global__ __launch_bounds__(256) void tsl_apply_kernel(float* __restrict__ P, i
 
 
 // As tsl_apply_kernel (w == 32), and the row's `rest` panel columns right of
-// the leaf take the update x -= l U12 (the rows' values already permuted).
-// Every workgroup solves U12 = L11^-1 xtop (the permuted top rows right of
-// the leaf) in LDS, one column per thread; workgroup 0 also stores it as the
-// top rows.  Four threads per row: each computes l and updates every fourth
-// column.
-constexpr int kApplyTpr = 4;
+// the leaf (at most 96, a multiple of 4) take the update x -= l U12 (the rows'
+// values already permuted).  64 rows per workgroup: wave 0 solves them, a row
+// per lane, while waves 1 and 2 solve U12 = L11^-1 xtop (the permuted top rows
+// right of the leaf), a column per lane; workgroup 0 also stores that as the
+// top rows.  Then each wave updates 16 rows by FP32 matrix products, C
+// requested at the start.  The solves' serial chains bound it (500 dependent
+// steps, L11\U11 read from LDS four values at a time); with four threads a
+// row, each solving it again and reading an LDS word per FMA, it took 23 us for
+// 16384 rows.
+constexpr int kApplyRows = 64;
 constexpr int kFuseRestMax = 96;  // panel columns right of a fused leaf (panels <= 128)
 __global__ __launch_bounds__(256) void tsl_apply_rest_kernel(float* __restrict__ P, int64_t ldp,
                                                              int m, const float* __restrict__ saved,
@@ -1472,116 +1495,140 @@ __global__ __launch_bounds__(256) void tsl_apply_rest_kernel(float* __restrict__
                                                              const float* __restrict__ xtop,
                                                              int rest) {
   __builtin_amdgcn_s_setprio(3);  // on the critical path (see tsl_kernel)
-  extern __shared__ float s_u12[];  // LW x rest
-  __shared__ float U[LW][LW + 1];
-  __shared__ float dinv[LW];
-  __shared__ int mpos[LW], msrc[LW];
-  __shared__ int s_nm;
-  const int tid = threadIdx.x;
-  for (int e = tid; e < LW * LW; e += 256) {
-    const int r = e / LW, c = e - r * LW;
-    U[r][c] = P[(int64_t)r * ldp + c];
-  }
-  if (tid == 0) s_nm = moved[0];
-  if (tid < LW) {
-    mpos[tid] = moved[1 + 2 * tid];
-    msrc[tid] = moved[2 + 2 * tid];
-  }
-  __syncthreads();
-  if (tid < LW) {
-    const float d = U[tid][tid];
-    dinv[tid] = d != 0.f ? 1.0f / d : 1.0f;  // a zero pivot leaves its column unscaled
-  }
-  for (int c = tid; c < rest; c += 256) {
-    float u[LW];
+  // row strides whose fragment reads (16 rows x 4 k, 16 columns x 4 k) and row
+  // reads (16 bytes a lane) fall on different banks
+  constexpr int LS = LW + 4, US = kFuseRestMax + 16, NTJ = kFuseRestMax / 16;
+  __shared__ __align__(16) float s_lu[LW][LW];          // L11\U11
+  __shared__ __align__(16) float s_l[kApplyRows * LS];  // the rows, then l
+  __shared__ float s_u12[LW * US];
+  __shared__ int s_m[2 * LW + 1];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lk = lane >> 4;
+  const int i0 = LW + blockIdx.x * kApplyRows;  // the workgroup's first row
+  const int nr = min(kApplyRows, m - i0);
+  // this lane's C: row i0 + 16 wave + l16, columns 16 t + 4 lk .. + 3 (past
+  // the last row or column: the last one's, never stored)
+  float* xrow = P + (int64_t)(i0 + min(16 * wave + l16, nr - 1)) * ldp + LW;
+  v4f x[NTJ];
 #pragma unroll
-    for (int i = 0; i < LW; ++i) {
-      float sum = xtop[i * rest + c];
+  for (int t = 0; t < NTJ; ++t)
+    x[t] = *reinterpret_cast<const v4f*>(xrow + min(16 * t + 4 * lk, rest - 4));
+  reinterpret_cast<v4f*>(&s_lu[0][0])[tid] =
+      *reinterpret_cast<const v4f*>(P + (int64_t)(tid >> 3) * ldp + 4 * (tid & 7));
+  const int nm = moved[0];
+  if (tid < 2 * nm) s_m[tid] = moved[1 + tid];
+  // the rows' 16-byte words, eight lanes a row
+  v4f a2[2];
 #pragma unroll
-      for (int k = 0; k < i; ++k) sum -= U[i][k] * u[k];
-      u[i] = sum;
-      s_u12[i * rest + c] = sum;
-    }
-    if (blockIdx.x == 0)
-#pragma unroll
-      for (int i = 0; i < LW; ++i) P[(int64_t)i * ldp + LW + c] = u[i];
+  for (int h = 0; h < 2; ++h) {
+    const int r = 32 * h + (tid >> 3);
+    a2[h] = *reinterpret_cast<const v4f*>(P + (int64_t)(i0 + min(r, nr - 1)) * ldp + 4 * (tid & 7));
   }
   __syncthreads();
-  const int q = tid % kApplyTpr;
-  const int i = LW + blockIdx.x * (256 / kApplyTpr) + tid / kApplyTpr;
-  if (i >= m) return;
-  int src = -1;
-  for (int k = 0; k < s_nm; ++k)
-    if (mpos[k] == i) src = msrc[k];
-  // 16-byte words throughout: the host fuses only panels whose rows start
-  // 16-byte aligned, with ldp and rest multiples of 4
-  float a[LW];
-  const v4f* arow = reinterpret_cast<const v4f*>(src >= 0 ? saved + src * LW
-                                                          : P + (int64_t)i * ldp);
 #pragma unroll
-  for (int c = 0; c < LW / 4; ++c) {
-    const v4f t = arow[c];
-    a[4 * c] = t.x;
-    a[4 * c + 1] = t.y;
-    a[4 * c + 2] = t.z;
-    a[4 * c + 3] = t.w;
+  for (int h = 0; h < 2; ++h) {
+    const int r = 32 * h + (tid >> 3);
+    int src = -1;
+    for (int k = 0; k < nm; ++k)
+      if (s_m[2 * k] == i0 + r) src = s_m[2 * k + 1];
+    if (src >= 0) a2[h] = reinterpret_cast<const v4f*>(saved + src * LW)[tid & 7];
+    *reinterpret_cast<v4f*>(&s_l[r * LS + 4 * (tid & 7)]) = a2[h];
   }
+  __syncthreads();
+  if (wave == 0) {
+    float a[LW];
+    v4f* row = reinterpret_cast<v4f*>(&s_l[lane * LS]);
 #pragma unroll
-  for (int k = 0; k < LW; ++k) {
-    const float x = a[k] * dinv[k];
-    a[k] = x;
-#pragma unroll
-    for (int c = k + 1; c < LW; ++c) a[c] -= x * U[k][c];
-  }
-  float* row = P + (int64_t)i * ldp;
-  if (q == 0) {
-#pragma unroll
-    for (int c = 0; c < LW / 4; ++c)
-      reinterpret_cast<v4f*>(row)[c] = v4f{a[4 * c], a[4 * c + 1], a[4 * c + 2], a[4 * c + 3]};
-  }
-  // the row's rest columns as 16-byte words q, q + 4, ... (rest is a
-  // multiple of 4; LDS reads of U12 stay 4-byte, broadcast across the 16
-  // rows of a wave)
-  v4f* xr = reinterpret_cast<v4f*>(row + LW);
-  const int nq = rest / 4;
-  for (int w0 = q; w0 < nq; w0 += kApplyTpr * 2) {
-    v4f x[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int w = w0 + kApplyTpr * t;
-      x[t] = w < nq ? xr[w] : v4f{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < LW / 4; ++c) {
+      const v4f t = row[c];
+      a[4 * c] = t.x;
+      a[4 * c + 1] = t.y;
+      a[4 * c + 2] = t.z;
+      a[4 * c + 3] = t.w;
     }
-#pragma unroll 4
+    // a zero pivot leaves its column unscaled
+    const float d = s_lu[lane & (LW - 1)][lane & (LW - 1)];
+    const float dinv = d != 0.f ? 1.0f / d : 1.0f;
+#pragma unroll
     for (int k = 0; k < LW; ++k) {
-      const float* uk = s_u12 + k * rest;
+      const float xk = a[k] * readlane_f(dinv, k);
+      a[k] = xk;
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const int c = 4 * min(w0 + kApplyTpr * t, nq - 1);
-        x[t][0] -= a[k] * uk[c];
-        x[t][1] -= a[k] * uk[c + 1];
-        x[t][2] -= a[k] * uk[c + 2];
-        x[t][3] -= a[k] * uk[c + 3];
+      for (int q = (k + 1) / 4; q < LW / 4; ++q) {
+        const v4f u = reinterpret_cast<const v4f*>(s_lu[k])[q];
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          if (4 * q + c > k) a[4 * q + c] -= xk * u[c];
       }
     }
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int w = w0 + kApplyTpr * t;
-      if (w < nq) xr[w] = x[t];
+    for (int c = 0; c < LW / 4; ++c)
+      row[c] = v4f{a[4 * c], a[4 * c + 1], a[4 * c + 2], a[4 * c + 3]};
+  } else if (wave < 3) {
+    const int c = tid - 64;
+    if (c < rest) {
+      float u[LW];
+#pragma unroll
+      for (int i = 0; i < LW; ++i) u[i] = xtop[i * rest + c];
+#pragma unroll
+      for (int i = 0; i < LW; ++i) {
+#pragma unroll
+        for (int q = 0; q < (i + 3) / 4; ++q) {
+          const v4f l = reinterpret_cast<const v4f*>(s_lu[i])[q];
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            if (4 * q + k < i) u[i] -= l[k] * u[4 * q + k];
+        }
+        s_u12[i * US + c] = u[i];
+      }
+      if (blockIdx.x == 0)
+#pragma unroll
+        for (int i = 0; i < LW; ++i) P[(int64_t)i * ldp + LW + c] = u[i];
+    } else if (c < kFuseRestMax) {
+#pragma unroll
+      for (int i = 0; i < LW; ++i) s_u12[i * US + c] = 0.f;
     }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int r = 32 * h + (tid >> 3);
+    if (r < nr)
+      *reinterpret_cast<v4f*>(P + (int64_t)(i0 + r) * ldp + 4 * (tid & 7)) =
+          *reinterpret_cast<const v4f*>(&s_l[r * LS + 4 * (tid & 7)]);
+  }
+  // x^T -= U12^T l^T: a lane's four results are four columns of one row
+  float lb[LW / 4];
+#pragma unroll
+  for (int k = 0; k < LW / 4; ++k) lb[k] = -s_l[(16 * wave + l16) * LS + 4 * k + lk];
+#pragma unroll
+  for (int t = 0; t < NTJ; ++t) {
+    if (16 * t >= rest) break;
+#pragma unroll
+    for (int k = 0; k < LW / 4; ++k)
+      x[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(s_u12[(4 * k + lk) * US + 16 * t + l16], lb[k],
+                                                  x[t], 0, 0, 0);
+    if (16 * wave + l16 < nr && 16 * t + 4 * lk < rest)
+      *reinterpret_cast<v4f*>(xrow + 16 * t + 4 * lk) = x[t];
   }
 }
 
 }  // namespace
 
 // Same outputs as leaf_lu; FP32 only.  Panels of up to 256 rows take the
-// partial-pivoting leaf.  Candidate groups are merged 8 at a time until at
-// most 32 remain for the final round (at most 8 for a one-wave final round
-// when the wide rounds are switched off).
+// partial-pivoting leaf.  The local round's groups: 256 rows up to 4096, 512
+// up to 8192, 1024 above, so that a final round over at most 512 candidates
+// follows (over 256 candidates for up to 8 groups); past 16384 rows, groups
+// are merged 16 at a time first.  With the wide rounds switched off every
+// round takes 256 rows.
 int leaf_lu_tournament(eamd_handle* h, float* P, int64_t ldp, int m, int w, int* piv,
                        int* lperm_n, int* lpos, int* lsrc, int* pperm_n, int* ppos, int* psrc,
                        int row0, int pnb, int* zero_col, int piv_offset, int* fz_global,
                        bool* fused) {
-  const int G1 = ceil_div(m, kTslBlock);
+  static const bool wide = env_int("EAMD_TSL_WIDE", 1) != 0;
+  const int cap = !wide || m <= 4096 ? 256 : (m <= 8192 ? 512 : 1024);
+  const int G1 = ceil_div(m, cap);
   // the leaf's interchanges on the other panel columns, the U rows right of
   // it and their update are done here too when w == 32 (the caller skips
   // its own)
@@ -1596,65 +1643,49 @@ int leaf_lu_tournament(eamd_handle* h, float* P, int64_t ldp, int m, int w, int*
     return kErrUnsupported;
   }
   void* base = nullptr;
-  // two candidate buffers (ping-pong between merge levels), counts, moved
-  // list and the saved rows
-  const size_t need = sizeof(int) * (2 * (size_t)G1 * LW + 2 * (size_t)G1 + 2 * LW + 8) +
+  // two candidate buffers (ping-pong between merge levels), moved list and the
+  // saved rows
+  const size_t need = sizeof(int) * (2 * (size_t)G1 * LW + 2 * LW + 8) +
                       sizeof(float) * LW * LW + sizeof(float) * LW * 256;
   EAMD_CHECK(h->ws.get(kWsTsl, need, &base));
   int* candA = static_cast<int*>(base);
   int* candB = candA + (size_t)G1 * LW;
-  int* nA = candB + (size_t)G1 * LW;
-  int* nB = nA + G1;
-  int* moved = nB + G1;
+  int* moved = candB + (size_t)G1 * LW;
   float* saved = reinterpret_cast<float*>(moved + 2 * LW + 8);
   float* xtop = saved + LW * LW;  // permuted top rows right of the leaf (fused)
   hipStream_t s = h->stream;
-  // Rounds: one wave per 256 rows, or per 512 rows in pairs when more than
-  // 32 groups would follow; merges of 8 groups while more than 32 remain;
-  // the final round in one workgroup (one wave for up to 8 groups, four
-  // waves for up to 32).
-  static const bool wide = env_int("EAMD_TSL_WIDE", 1) != 0;
-  const int fan1 = wide ? 4 * kTslFan : kTslFan;
-  int G;
-  if (wide && G1 > fan1) {
-    G = ceil_div(m, 2 * kTslBlock);
-    hipLaunchKernelGGL((tsl_kernel<0, 2>), dim3(G), dim3(128), 0, s, P, ldp, m, w, nullptr,
-                       nullptr, 0, candA, nA, saved, moved, piv, lperm_n, lpos, lsrc, pperm_n,
-                       ppos, psrc, row0, pnb, zero_col, piv_offset, fz_global, 0, xtop);
-  } else {
-    G = G1;
-    hipLaunchKernelGGL((tsl_kernel<0, 1>), dim3(G), dim3(64), 0, s, P, ldp, m, w, nullptr,
-                       nullptr, 0, candA, nA, saved, moved, piv, lperm_n, lpos, lsrc, pperm_n,
-                       ppos, psrc, row0, pnb, zero_col, piv_offset, fz_global, 0, xtop);
-  }
-  int *cin = candA, *nin = nA, *cout = candB, *nout = nB;
-  while (G > fan1) {
-    const int Gn = ceil_div(G, kTslFan);
-    hipLaunchKernelGGL((tsl_kernel<2, 1>), dim3(Gn), dim3(64), 0, s, P, ldp, m, w, cin, nin, G,
-                       cout, nout, saved, moved, piv, lperm_n, lpos, lsrc, pperm_n, ppos, psrc,
-                       row0, pnb, zero_col, piv_offset, fz_global, 0, xtop);
+  int *cin = nullptr, *cout = candA, *spare = candB;
+  int G = G1, n = 0;  // groups, and candidates in them
+#define EAMD_TSL(MODE, CAP, BLOCKS)                                                           \
+  hipLaunchKernelGGL((tsl_kernel<MODE, CAP>), dim3(BLOCKS),                                   \
+                     dim3(64 * (Tsl<CAP>::NW + (MODE == 1))), 0, s, P, ldp, m, w, cin, n, cout, \
+                     saved, moved, piv, lperm_n, lpos, lsrc, pperm_n, ppos, psrc, row0, pnb,  \
+                     zero_col, piv_offset, fz_global, fuse ? 1 : 0, xtop)
+  if (cap == 256) EAMD_TSL(0, 256, G);
+  else if (cap == 512) EAMD_TSL(0, 512, G);
+  else EAMD_TSL(0, 1024, G);
+  n = (G - 1) * w + std::min(w, m - (G - 1) * cap);
+  cin = cout;
+  cout = spare;
+  spare = cin;
+  const int fan = wide ? 512 / LW : 256 / LW;
+  while (G > fan) {
+    const int Gn = ceil_div(G, fan);
+    if (wide) EAMD_TSL(2, 512, Gn);
+    else EAMD_TSL(2, 256, Gn);
+    n = (Gn - 1) * w + std::min(w, n - (Gn - 1) * fan * w);
     G = Gn;
-    std::swap(cin, cout);
-    std::swap(nin, nout);
+    cin = cout;
+    cout = spare;
+    spare = cin;
   }
-  if (G > kTslFan)
-    hipLaunchKernelGGL((tsl_kernel<1, 4>), dim3(1), dim3(256), 0, s, P, ldp, m, w, cin, nin, G,
-                       cout, nout, saved, moved, piv, lperm_n, lpos, lsrc, pperm_n, ppos, psrc,
-                       row0, pnb, zero_col, piv_offset, fz_global, fuse ? 1 : 0, xtop);
-  else
-    hipLaunchKernelGGL((tsl_kernel<1, 1>), dim3(1), dim3(64), 0, s, P, ldp, m, w, cin, nin, G,
-                       cout, nout, saved, moved, piv, lperm_n, lpos, lsrc, pperm_n, ppos, psrc,
-                       row0, pnb, zero_col, piv_offset, fz_global, fuse ? 1 : 0, xtop);
+  if (G > 256 / LW) EAMD_TSL(1, 512, 1);
+  else EAMD_TSL(1, 256, 1);
+#undef EAMD_TSL
   const int rest = pnb - row0 - w;
   if (fuse && rest > 0) {
-    static bool attr_set = false;
-    if (!attr_set) {
-      EAMD_HIP(hipFuncSetAttribute((const void*)tsl_apply_rest_kernel,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024));
-      attr_set = true;
-    }
-    hipLaunchKernelGGL(tsl_apply_rest_kernel, dim3(ceil_div(m - w, 256 / kApplyTpr)), dim3(256),
-                       sizeof(float) * LW * rest, s, P, ldp, m, saved, moved, xtop, rest);
+    hipLaunchKernelGGL(tsl_apply_rest_kernel, dim3(ceil_div(m - w, kApplyRows)), dim3(256), 0, s,
+                       P, ldp, m, saved, moved, xtop, rest);
   } else if (m > w) {
     if (w == LW)
       hipLaunchKernelGGL(tsl_apply_kernel<true>, dim3(ceil_div(m - w, 256)), dim3(256), 0, s, P,
