@@ -16,7 +16,7 @@
 // transposed so a lane holds four adjacent columns of a row; FP64 for the
 // refactor pass).  With more than one wave the next panel's columns are
 // updated first and wave 0 factors that panel while the other waves update
-// the rest.  The solves (right-looking in 64-row blocks, 16 lanes per row)
+// the rest.  The solves (right-looking in 64-row blocks, by matrix products)
 // and the refinement steps (residual B - A X in FP64 from the original A)
 // stay in the same workgroup.  The workgroup size (64, 128 or 256 threads)
 // is chosen per 16-wide size bucket by timing on synthetic systems, once per
@@ -36,6 +36,7 @@ constexpr int kMaxLuN = 256;
 constexpr int PB = 16;       // panel width = the MFMA k-depth used per trailing update
 constexpr int kMaxRhs = 8;
 constexpr int DB = 64;       // diagonal block of the triangular solves (one wave)
+constexpr int kDiagLd = DB + 4;  // FP32: 16-byte rows on different banks
 constexpr int kMaxIter = 10;
 constexpr double kTol = 1e-14;
 
@@ -114,7 +115,7 @@ struct LuSmem {
   static constexpr int kPanel = NMAX * (PB + 1);
   static constexpr int kU = PB * (NMAX + 1);
   // solves: the diagonal triangle, the right-hand sides and the residual
-  static constexpr int kDiag = DB * (DB + 1);
+  static constexpr int kDiag = DB * (sizeof(TF) == 4 ? kDiagLd : DB + 1);
   static constexpr int kVec = NMAX * kMaxRhs;
   static constexpr int kWords = (kPanel + kU) > (kDiag + 2 * kVec) ? (kPanel + kU)
                                                                    : (kDiag + 2 * kVec);
@@ -234,8 +235,8 @@ __device__ __forceinline__ void load_rows(const TF* __restrict__ W, int n, int b
   }
 }
 
-// Forward (unit lower, FORWARD=true) or backward (upper) substitution of the
-// NR (>= nrhs) columns y[r * kMaxRhs + q] against the factors in the
+// The FP64 refactor pass's solves: forward (unit lower, FORWARD=true) or
+// backward (upper) substitution of the NR (>= nrhs) columns y[r * kMaxRhs + q] against the factors in the
 // row-major W, right-looking in blocks of DB rows.  The block's strict
 // triangle is staged in LDS (zero-padded to DB, with U's reciprocal diagonal
 // in column DB) and solved by wave 0, lanes over rows, the DB steps unrolled
@@ -351,6 +352,201 @@ __device__ __forceinline__ void tri_solve(const TF* __restrict__ W, int n, TF* y
     }
     __syncthreads();
   }
+}
+
+// acc[h] += (lane T of each row of sixteen of x[h]) * l.  The wait states
+// cover the VALU writes of x just before.
+template <int T, int H>
+__device__ __forceinline__ void fmac_lane(float (&acc)[H], const float (&x)[H], float l) {
+  static_assert(H == 1 || H == 2, "four or eight right-hand sides");
+  if constexpr (H == 1)
+    asm volatile("s_nop 1\n\tv_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+                 : "+v"(acc[0])
+                 : "v"(x[0]), "v"(l), "n"(T));
+  else
+    asm volatile("s_nop 1\n\tv_fmac_f32_dpp %0, %2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %1, %3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+                 : "+v"(acc[0]), "+v"(acc[1])
+                 : "v"(x[0]), "v"(x[1]), "v"(l), "n"(T));
+}
+// as above with x = acc (a lane above T adds a zero)
+template <int T, int H>
+__device__ __forceinline__ void fmac_lane_self(float (&acc)[H], float l) {
+  if constexpr (H == 1)
+    asm volatile("s_nop 1\n\tv_fmac_f32_dpp %0, %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf"
+                 : "+v"(acc[0])
+                 : "v"(l), "n"(T));
+  else
+    asm volatile("s_nop 1\n\tv_fmac_f32_dpp %0, %0, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %1, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+                 : "+v"(acc[0]), "+v"(acc[1])
+                 : "v"(l), "n"(T));
+}
+template <int T, int H, bool FORWARD>
+__device__ __forceinline__ void tri16(float (&acc)[H], const float (&l)[16], float rd) {
+  if constexpr (FORWARD && T < 15) {
+    fmac_lane_self<T, H>(acc, l[T]);
+    tri16<T + 1, H, FORWARD>(acc, l, rd);
+  } else if constexpr (!FORWARD && T > 0) {
+    float z[H];
+#pragma unroll
+    for (int h = 0; h < H; ++h) z[h] = acc[h] * rd;
+    fmac_lane<T, H>(acc, z, l[T]);
+    tri16<T - 1, H, FORWARD>(acc, l, rd);
+  }
+}
+
+// Forward (unit lower, FORWARD=true) or backward (upper) substitution in FP32
+// of the NR (4 or 8) columns y[r * kMaxRhs + q] against the factors in the
+// row-major W, right-looking in blocks of DB rows.  The diagonal block is
+// staged in LDS (its loads requested a block ahead) and solved by wave 0 in
+// sub-blocks of 16 rows: lane (row, q) takes a row of one right-hand side,
+// the solved value comes by the FMA's lane broadcast, and the block's other
+// rows take the sub-block by 16x16x4 products.  Every row beyond the block
+// then takes it the same way, 16 rows a tile, by all waves: lane (l16, lk)
+// loads columns 16 c + 4 lk .. + 3 of row l16 in one 16-byte word, and
+// product (c, j) pairs element j of those words with the same rows of y.
+// Only NR of a product's 16 columns are used; even so a tile costs half of
+// what FMAs and sums over 16 lanes cost, and the diagonal's chain is 16
+// fused steps per sub-block instead of a readlane and an FMA per column and
+// step.  65,536 systems of 16..256, 4 right-hand sides: the solves fell from
+// 30 to 15 percent of a workgroup's cycles, 43.7 to 39.9 ms in all.
+template <int NT, bool FORWARD, int NR>
+__device__ __forceinline__ void tri_solve_f32(const float* __restrict__ W, int n, float* y,
+                                              float* diag, int tid0) {
+  constexpr int NW = NT / 64, H = NR / 4, LD = kDiagLd, PER = DB * DB / 4 / NT;
+  const int nblk = (n + DB - 1) / DB;
+  const int wave = __builtin_amdgcn_readfirstlane(tid0 >> 6);
+  // the diagonal block's 16-byte words, tid + k NT (row, word); past the
+  // matrix: its last row and columns (masked where they are used)
+  v4f dg[PER];
+  auto load_diag = [&](int bb, int tid) {
+    const int b0 = (FORWARD ? bb : nblk - 1 - bb) * DB, bn = min(DB, n - b0);
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int e = tid + k * NT, c = 4 * (e & 15);
+      const float* row = W + min(b0 + (e >> 4), n - 1) * n + b0;
+      if (bn == DB) {
+        dg[k] = *reinterpret_cast<const f4u*>(row + c);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dg[k][j] = row[min(c + j, bn - 1)];
+      }
+    }
+  };
+  auto store_diag = [&](int tid) {
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int e = tid + k * NT;
+      *reinterpret_cast<v4f*>(diag + (e >> 4) * LD + 4 * (e & 15)) = dg[k];
+    }
+  };
+  load_diag(0, tid0);
+  store_diag(tid0);
+#pragma unroll 1
+  for (int bb = 0; bb < nblk; ++bb) {
+    const int tid = opaque(tid0), lane = tid & 63, l16 = lane & 15, lk = lane >> 4;
+    const int b0 = (FORWARD ? bb : nblk - 1 - bb) * DB, bn = min(DB, n - b0);
+    const int r_lo = FORWARD ? b0 + bn : 0, r_hi = FORWARD ? n : b0;
+    const int tiles = (r_hi - r_lo + 15) / 16;
+    const bool more = bb + 1 < nblk;
+    __syncthreads();
+    if (more) load_diag(bb + 1, tid);
+    // (rows past the matrix: its last row, into rows of y nobody reads)
+    v4f a[4];
+    auto load_tile = [&](int t) {
+      const float* p = W + min(r_lo + 16 * t + l16, n - 1) * n + b0 + 4 * lk;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) a[c] = *reinterpret_cast<const f4u*>(p + 16 * c);
+    };
+    if (wave < tiles) load_tile(wave);
+    if (wave == 0) {
+      const int ns = (bn + 15) / 16;
+#pragma unroll 1
+      for (int ss = 0; ss < ns; ++ss) {
+        const int s = FORWARD ? ss : ns - 1 - ss, s0 = 16 * s;
+        const bool in = s0 + l16 < bn;
+        float l[16], rd = 1.f, acc[H];
+        const float* lr = diag + (s0 + l16) * LD + s0;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const v4f x = *reinterpret_cast<const v4f*>(lr + 4 * c);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int t = 4 * c + j;
+            const bool keep = FORWARD ? t < l16 : t > l16 && s0 + t < bn;
+            l[t] = keep && in ? -x[j] : 0.f;
+          }
+        }
+        if (!FORWARD && in) rd = 1.f / lr[l16];
+        float* yr = y + (b0 + s0 + l16) * kMaxRhs + lk;
+#pragma unroll
+        for (int h = 0; h < H; ++h) acc[h] = in ? yr[4 * h] : 0.f;
+        tri16<FORWARD ? 0 : 15, H, FORWARD>(acc, l, rd);
+        if (!FORWARD)
+#pragma unroll
+          for (int h = 0; h < H; ++h) acc[h] *= rd;
+        if (in) {
+#pragma unroll
+          for (int h = 0; h < H; ++h) yr[4 * h] = acc[h];
+        }
+        asm volatile("" ::: "memory");  // a wave's LDS accesses execute in order
+        // the block's other rows
+        float b[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int k = s0 + 4 * lk + j;
+          const float x = y[(b0 + k) * kMaxRhs + (l16 & (kMaxRhs - 1))];
+          b[j] = l16 < NR && k < bn ? -x : 0.f;
+        }
+#pragma unroll 1
+        for (int u = FORWARD ? s + 1 : 0; u < (FORWARD ? ns : s); ++u) {
+          const v4f x = *reinterpret_cast<const v4f*>(diag + (16 * u + l16) * LD + s0 + 4 * lk);
+          float* c = y + (b0 + 16 * u + 4 * lk) * kMaxRhs + (l16 & (kMaxRhs - 1));
+          v4f d;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) d[r] = c[r * kMaxRhs];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) d = mfma16x4(s0 + 4 * lk + j < bn ? x[j] : 0.f, b[j], d);
+          if (l16 < NR) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) c[r * kMaxRhs] = d[r];
+          }
+        }
+        asm volatile("" ::: "memory");
+      }
+    }
+    __syncthreads();
+    if (more) store_diag(tid);
+    if (wave < tiles) {
+      float b[4][4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int k = 16 * c + 4 * lk + j;
+          const float x = y[(b0 + k) * kMaxRhs + (l16 & (kMaxRhs - 1))];
+          b[c][j] = l16 < NR && k < bn ? -x : 0.f;
+        }
+#pragma unroll 1
+      for (int t = wave; t < tiles; t += NW) {
+        float* c0 = y + (r_lo + 16 * t + 4 * lk) * kMaxRhs + (l16 & (kMaxRhs - 1));
+        v4f d;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) d[r] = c0[r * kMaxRhs];
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) d = mfma16x4(a[c][j], b[c][j], d);
+        if (t + NW < tiles) load_tile(t + NW);
+        if (l16 < NR) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) c0[r * kMaxRhs] = d[r];
+        }
+      }
+    }
+  }
+  __syncthreads();
 }
 
 // u[j - C] = P[ks][j] of lane pl for j = C..PB-1, ks uniform: one readlane
@@ -955,13 +1151,18 @@ __global__ __launch_bounds__(NT, sizeof(TF) == 8 ? 1 : (NT == 256 ? 4 : (NT == 1
           if (e0 + k * NT < n * kMaxRhs) y[e0 + k * NT] = (TF)v[k];
       }
       __syncthreads();
-      if (nrhs <= 4) {
-        tri_solve<TF, NT, true, 4>(W, n, y, diag, tid);
-        tri_solve<TF, NT, false, 4>(W, n, y, diag, tid);
-      } else {
-        tri_solve<TF, NT, true, kMaxRhs>(W, n, y, diag, tid);
-        tri_solve<TF, NT, false, kMaxRhs>(W, n, y, diag, tid);
-      }
+      auto solve = [&](auto nr) {
+        constexpr int NR = decltype(nr)::value;
+        if constexpr (sizeof(TF) == 4) {
+          tri_solve_f32<NT, true, NR>(W, n, y, diag, tid);
+          tri_solve_f32<NT, false, NR>(W, n, y, diag, tid);
+        } else {
+          tri_solve<TF, NT, true, NR>(W, n, y, diag, tid);
+          tri_solve<TF, NT, false, NR>(W, n, y, diag, tid);
+        }
+      };
+      if (nrhs <= 4) solve(std::integral_constant<int, 4>{});
+      else solve(std::integral_constant<int, kMaxRhs>{});
       // X = the solution (first pass) or X + the correction, written to X and
       // staged in LDS as FP64 for the residual (in the diagonal-block area,
       // which the solves no longer use); eight entries per thread, the old
