@@ -5,19 +5,19 @@
 // tolerance are refactored in FP64 by a second launch.
 //
 // MI355X mapping.  One workgroup per system (n <= 256), systems taken in
-// descending size from the plan's order so the largest start first.  The
-// workgroup converts its FP64 column-major A_i into a row-major working copy
-// W_i (row interchanges are then contiguous), and runs a right-looking
-// blocked LU with 16-column panels.  A panel is factored by wave 0 in its
-// registers (pivot search by DPP wave reductions, interchanges as swapped
-// row positions, the pivot row broadcast by readlane); the interchanges are
-// applied to the other columns, U12 is solved against the unit lower L11,
-// and the trailing update A22 -= L21 U12 runs as 16x16x4 MFMA tiles (FP32,
-// transposed so a lane holds four adjacent columns of a row; FP64 for the
-// refactor pass).  With more than one wave the next panel's columns are
-// updated first and wave 0 factors that panel while the other waves update
-// the rest.  The solves (right-looking in 64-row blocks, by matrix products)
-// and the refinement steps (residual B - A X in FP64 from the original A)
+// descending size from the plan's order so the largest start first.  The FP32
+// factorization is left-looking in 16-column panels with 16x16x4 matrix
+// products, rows addressed through the permutation instead of moved
+// (factor_f32); the FP64 refactor pass converts A_i into a row-major working
+// copy W_i (row interchanges are then contiguous) and runs a right-looking
+// blocked LU on it: a panel is factored by wave 0 in its registers (pivot
+// search by DPP wave reductions, interchanges as swapped row positions, the
+// pivot row broadcast by readlane), the interchanges are applied to the other
+// columns, U12 is solved against the unit lower L11, and the trailing update
+// A22 -= L21 U12 runs as 16x16x4 tiles, the next panel's columns first, so
+// that wave 0 factors that panel while the other waves update the rest.  The
+// solves (right-looking in 64-row blocks, by matrix products in FP32) and the
+// refinement steps (residual B - A X in FP64 from the original A)
 // stay in the same workgroup.  The workgroup size (64, 128 or 256 threads)
 // is chosen per 16-wide size bucket by timing on synthetic systems, once per
 // process.
@@ -37,8 +37,14 @@ constexpr int PB = 16;       // panel width = the MFMA k-depth used per trailing
 constexpr int kMaxRhs = 8;
 constexpr int DB = 64;       // diagonal block of the triangular solves (one wave)
 constexpr int kDiagLd = DB + 4;  // FP32: 16-byte rows on different banks
+constexpr int kPanelLd = PB + 4;  // FP32 panel rows: 16-byte words on different banks
 constexpr int kMaxIter = 10;
 constexpr double kTol = 1e-14;
+// From the FP32 factor the refinement goes on below kTol while a step still
+// gains: one step from this factor leaves most systems between the two, and
+// the next costs a pass over A (65,536 systems of 16..256: 26.1 ms and an
+// error of 8e-16; 23.2 ms and 2e-14 with kTol alone).
+constexpr double kDone = 1e-15;
 
 __device__ __forceinline__ v4f mfma16x4(float a, float b, v4f c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -46,21 +52,8 @@ __device__ __forceinline__ v4f mfma16x4(float a, float b, v4f c) {
 __device__ __forceinline__ v4d mfma16x4(double a, double b, v4d c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
-template <typename T>
-struct Acc4;
-template <>
-struct Acc4<float> {
-  typedef v4f type;
-};
-template <>
-struct Acc4<double> {
-  typedef v4d type;
-};
-// row of accumulator register r in lane l (column is l % 16)
-template <typename T>
-__device__ __forceinline__ int acc_row(int l, int r) {
-  return sizeof(T) == 4 ? 4 * (l >> 4) + r : (l >> 4) + 4 * r;
-}
+// row of the FP64 accumulator's register r in lane l (column is l % 16)
+__device__ __forceinline__ int acc_row(int l, int r) { return (l >> 4) + 4 * r; }
 
 template <int CTRL>
 __device__ __forceinline__ double dpp_d(double x) {
@@ -117,8 +110,10 @@ struct LuSmem {
   // solves: the diagonal triangle, the right-hand sides and the residual
   static constexpr int kDiag = DB * (sizeof(TF) == 4 ? kDiagLd : DB + 1);
   static constexpr int kVec = NMAX * kMaxRhs;
-  static constexpr int kWords = (kPanel + kU) > (kDiag + 2 * kVec) ? (kPanel + kU)
-                                                                   : (kDiag + 2 * kVec);
+  // the FP32 factorization: the panel's rows and two U blocks
+  static constexpr int kLeft = (NMAX + 2 * PB) * kPanelLd;
+  static constexpr int kFactor = sizeof(TF) == 4 ? kLeft : kPanel + kU;
+  static constexpr int kWords = kFactor > (kDiag + 2 * kVec) ? kFactor : (kDiag + 2 * kVec);
 };
 
 // |x| with a NaN mapped to +infinity, so maxima keep it
@@ -398,7 +393,7 @@ __device__ __forceinline__ void tri16(float (&acc)[H], const float (&l)[16], flo
 
 // Forward (unit lower, FORWARD=true) or backward (upper) substitution in FP32
 // of the NR (4 or 8) columns y[r * kMaxRhs + q] against the factors in the
-// row-major W, right-looking in blocks of DB rows.  The diagonal block is
+// row-major W (row r of the factors is row perm[r] of W), right-looking in blocks of DB rows.  The diagonal block is
 // staged in LDS (its loads requested a block ahead) and solved by wave 0 in
 // sub-blocks of 16 rows: lane (row, q) takes a row of one right-hand side,
 // the solved value comes by the FMA's lane broadcast, and the block's other
@@ -412,8 +407,8 @@ __device__ __forceinline__ void tri16(float (&acc)[H], const float (&l)[16], flo
 // step.  65,536 systems of 16..256, 4 right-hand sides: the solves fell from
 // 30 to 15 percent of a workgroup's cycles, 43.7 to 39.9 ms in all.
 template <int NT, bool FORWARD, int NR>
-__device__ __forceinline__ void tri_solve_f32(const float* __restrict__ W, int n, float* y,
-                                              float* diag, int tid0) {
+__device__ __forceinline__ void tri_solve_f32(const float* __restrict__ W, int n,
+                                              const int* perm, float* y, float* diag, int tid0) {
   constexpr int NW = NT / 64, H = NR / 4, LD = kDiagLd, PER = DB * DB / 4 / NT;
   const int nblk = (n + DB - 1) / DB;
   const int wave = __builtin_amdgcn_readfirstlane(tid0 >> 6);
@@ -425,7 +420,7 @@ __device__ __forceinline__ void tri_solve_f32(const float* __restrict__ W, int n
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
       const int e = tid + k * NT, c = 4 * (e & 15);
-      const float* row = W + min(b0 + (e >> 4), n - 1) * n + b0;
+      const float* row = W + perm[min(b0 + (e >> 4), n - 1)] * n + b0;
       if (bn == DB) {
         dg[k] = *reinterpret_cast<const f4u*>(row + c);
       } else {
@@ -455,7 +450,7 @@ __device__ __forceinline__ void tri_solve_f32(const float* __restrict__ W, int n
     // (rows past the matrix: its last row, into rows of y nobody reads)
     v4f a[4];
     auto load_tile = [&](int t) {
-      const float* p = W + min(r_lo + 16 * t + l16, n - 1) * n + b0 + 4 * lk;
+      const float* p = W + perm[min(r_lo + 16 * t + l16, n - 1)] * n + b0 + 4 * lk;
 #pragma unroll
       for (int c = 0; c < 4; ++c) a[c] = *reinterpret_cast<const f4u*>(p + 16 * c);
     };
@@ -503,14 +498,12 @@ __device__ __forceinline__ void tri_solve_f32(const float* __restrict__ W, int n
         for (int u = FORWARD ? s + 1 : 0; u < (FORWARD ? ns : s); ++u) {
           const v4f x = *reinterpret_cast<const v4f*>(diag + (16 * u + l16) * LD + s0 + 4 * lk);
           float* c = y + (b0 + 16 * u + 4 * lk) * kMaxRhs + (l16 & (kMaxRhs - 1));
-          v4f d;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) d[r] = c[r * kMaxRhs];
+          v4f d = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int j = 0; j < 4; ++j) d = mfma16x4(s0 + 4 * lk + j < bn ? x[j] : 0.f, b[j], d);
           if (l16 < NR) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) c[r * kMaxRhs] = d[r];
+            for (int r = 0; r < 4; ++r) c[r * kMaxRhs] += d[r];
           }
         }
         asm volatile("" ::: "memory");
@@ -531,17 +524,20 @@ __device__ __forceinline__ void tri_solve_f32(const float* __restrict__ W, int n
 #pragma unroll 1
       for (int t = wave; t < tiles; t += NW) {
         float* c0 = y + (r_lo + 16 * t + 4 * lk) * kMaxRhs + (l16 & (kMaxRhs - 1));
-        v4f d;
+        // (sums of 32 products each, then one addition to y: the rounding of
+        // a sum over 64, and a shorter chain of products)
+        v4f d = {0.f, 0.f, 0.f, 0.f}, e = d;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) d[r] = c0[r * kMaxRhs];
+        for (int c = 0; c < 2; ++c)
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) d = mfma16x4(a[c][j], b[c][j], d);
+          for (int j = 0; j < 4; ++j) {
+            d = mfma16x4(a[c][j], b[c][j], d);
+            e = mfma16x4(a[c + 2][j], b[c + 2][j], e);
+          }
         if (t + NW < tiles) load_tile(t + NW);
         if (l16 < NR) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) c0[r * kMaxRhs] = d[r];
+          for (int r = 0; r < 4; ++r) c0[r * kMaxRhs] += d[r] + e[r];
         }
       }
     }
@@ -634,6 +630,265 @@ struct PanelCols<TF, NS, PB> {
   __device__ __forceinline__ static void run(TF (&)[NS][PB], int (&)[NS], int, int, int, int,
                                              int*) {}
 };
+
+// Maximum of a 32-bit key over the 64 lanes of a wave: within each row of
+// sixteen by DPP maxima, then the rows' maxima read as uniform values.
+__device__ __forceinline__ unsigned wave_max_key(unsigned k) {
+  k = max(k, (unsigned)__builtin_amdgcn_mov_dpp((int)k, 0xB1, 0xf, 0xf, false));
+  k = max(k, (unsigned)__builtin_amdgcn_mov_dpp((int)k, 0x4E, 0xf, 0xf, false));
+  k = max(k, (unsigned)__builtin_amdgcn_mov_dpp((int)k, 0x141, 0xf, 0xf, false));
+  k = max(k, (unsigned)__builtin_amdgcn_mov_dpp((int)k, 0x140, 0xf, 0xf, false));
+  return max(max((unsigned)__builtin_amdgcn_readlane((int)k, 0),
+                 (unsigned)__builtin_amdgcn_readlane((int)k, 16)),
+             max((unsigned)__builtin_amdgcn_readlane((int)k, 32),
+                 (unsigned)__builtin_amdgcn_readlane((int)k, 48)));
+}
+
+// Column step C of the FP32 panel in one wave's registers: slot lane + 64 k is
+// the panel's row of that number, em[k] is all ones while it is a candidate
+// and st[k] the step that picked it.  The key is |a| with its eight low
+// mantissa bits replaced by 255 - slot: one integer maximum names the pivot,
+// equal magnitudes go to the first row, and scores within 2^-15 count as
+// equal (multipliers up to 1 + 2^-15; the refinement judges the factor).
+template <int NS, int C>
+__device__ __forceinline__ void panel_col_f32(float (&P)[NS][PB], unsigned (&em)[NS],
+                                              int (&st)[NS], int lane) {
+  // (columns are scheduled one by one: register pressure)
+  __builtin_amdgcn_sched_barrier(0);
+  unsigned key = 0;
+#pragma unroll
+  for (int k = 0; k < NS; ++k)
+    key = max(key, ((__float_as_uint(P[k][C]) & 0x7fffff00u) | (255u - lane - 64u * k)) & em[k]);
+  const int q = 255 - (int)(wave_max_key(key) & 255u), ks = q >> 6, pl = q & 63;
+  float u[PB - C];
+  PivotRow<float, NS, C, 0>::get(P, ks, pl, u);
+#pragma unroll
+  for (int k = 0; k < NS; ++k) {
+    const bool sel = lane + 64 * k == q && em[k];
+    em[k] = sel ? 0u : em[k];
+    st[k] = sel ? C : st[k];
+  }
+  // a zero pivot leaves a column of zeros
+  const float pv = u[0], rp = pv != 0.f ? 1.f / pv : 0.f;
+#pragma unroll
+  for (int k = 0; k < NS; ++k) {
+    const float l = P[k][C] * rp;
+    const float le = __uint_as_float(__float_as_uint(l) & em[k]);
+    P[k][C] = em[k] ? l : P[k][C];
+    // (selected now, not when the row is stored: both sides and the masks of
+    // every column would stay live)
+    asm volatile("" : "+v"(P[k][C]), "+v"(em[k]), "+v"(st[k]));
+#pragma unroll
+    for (int j = C + 1; j < PB; ++j) P[k][j] -= le * u[j - C];
+  }
+}
+// The panel's columns, four at a time (past the last column no candidate is
+// left and nothing that is kept changes): a branch per column costs registers
+// where its sides meet.
+template <int NS, int C>
+__device__ __forceinline__ void panel_cols_f32(float (&P)[NS][PB], unsigned (&em)[NS],
+                                               int (&st)[NS], int lane, int pb) {
+  if constexpr (C < PB) {
+    if (C < pb) {
+      panel_col_f32<NS, C>(P, em, st, lane);
+      panel_col_f32<NS, C + 1>(P, em, st, lane);
+      panel_col_f32<NS, C + 2>(P, em, st, lane);
+      panel_col_f32<NS, C + 3>(P, em, st, lane);
+      panel_cols_f32<NS, C + 4>(P, em, st, lane, pb);
+    }
+  }
+}
+
+// x[r] += (lane T of each row of sixteen of x[r]) * l for the four columns r,
+// T = 0 .. 14: the unit lower solve of 16 rows (lane l16: row l16, l[t] = minus
+// its strict lower part), columns in registers.
+template <int T>
+__device__ __forceinline__ void unit16(v4f& x, const float (&l)[16]) {
+  if constexpr (T < 15) {
+    float x0 = x[0], x1 = x[1], x2 = x[2], x3 = x[3];
+    asm volatile("s_nop 1\n\tv_fmac_f32_dpp %0, %0, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %1, %1, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %2, %2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %3, %3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+                 : "+v"(x0), "+v"(x1), "+v"(x2), "+v"(x3)
+                 : "v"(l[T]), "n"(T));
+    x = v4f{x0, x1, x2, x3};
+    unit16<T + 1>(x, l);
+  }
+}
+
+// The FP32 factorization: left-looking in panels of 16 columns, rows never
+// moved.  Row r of the factors is row perm[r] of W (and of A), so an
+// interchange is two entries of perm; a panel is read from A's columns in the
+// order of perm (tile t, wave t % NW: lane (l16, lk) holds columns 4 lk .. + 3
+// of row 16 t + l16), and takes the
+// earlier panels one 16-row block of U at a time: the block's wave solves it
+// against L's diagonal block, it goes round through LDS, and every tile below
+// takes its four products with L read from W.  The finished rows then go
+// through LDS to wave 0, a row or more per lane, which factors the panel.
+// A is subtracted from in FP64, so its own rounding comes after the products'
+// sum.  What decides: W is written once and L read once per panel, a quarter
+// of what updating the trailing matrix in place moves (67 + 52 GB for 65,536
+// systems of 16..256 then), and the copy of A, the row moves and the U rows'
+// pass over W are gone: 39.9 ms right-looking, 26.1 so.  What bounds it now:
+// the chain of U blocks, a barrier each, and the panel's columns, one after
+// the other, with three more workgroups on the CU to fill in.
+template <int NT, int NMAX>
+__device__ __forceinline__ void factor_f32(const double* __restrict__ As, float* W, int n,
+                                           int* perm, float* smem, int wave) {
+  constexpr int NW = NT / 64, MT = (NMAX / 16 + NW - 1) / NW, NS = NMAX / 64, PL = kPanelLd;
+  float* Pn = smem;             // the panel's rows
+  float* Ub = smem + NMAX * PL; // minus two blocks of U, k by column
+  const int nt = (n + 15) / 16;
+  for (int r = thread_index(wave); r <= n; r += NT) perm[r] = r;
+  __syncthreads();
+#pragma unroll 1
+  for (int k0 = 0; k0 < n; k0 += PB) {
+    const int lane = thread_index(0), l16 = lane & 15, lk = lane >> 4;
+    const int kb = k0 / PB, pb = min(PB, n - k0);
+    // tiles of rows past the matrix repeat its last row, columns past it its
+    // last column (never candidates, never stored)
+    unsigned wr[MT];  // byte offset in W of the row's columns 4 lk ..
+    char* const Wc = reinterpret_cast<char*>(W);
+    v4f c[MT], a[MT];  // minus the sum of the products; L's next operand
+    double ad[MT][4];  // A's entries
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int t = i * NW + wave;
+      const int o = perm[min(16 * t + l16, n - 1)];
+      wr[i] = 4u * (unsigned)(o * n + 4 * lk);
+      c[i] = a[i] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int r = 0; r < 4; ++r) ad[i][r] = 0.0;
+      if (t < nt) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          ad[i][r] = *reinterpret_cast<const double*>(
+              reinterpret_cast<const char*>(As) +
+              8u * (unsigned)(o + min(k0 + 4 * lk + r, n - 1) * n));
+      }
+      if (kb > 0 && t > 0 && t < nt) a[i] = *reinterpret_cast<const f4u*>(Wc + wr[i]);
+    }
+    // the next diagonal block of L this wave solves against
+    v4f lb[4] = {};
+    auto load_lb = [&](int b) {
+      const unsigned p = 4u * (unsigned)(perm[16 * b + l16] * n);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) lb[q] = *reinterpret_cast<const f4u*>(Wc + 64 * b + 16 * q + p);
+    };
+    if (wave < kb) load_lb(wave);
+#pragma unroll 1
+    for (int b = 0; b < kb; ++b) {
+      float* ub = Ub + (b & 1) * PB * PL;
+      if (b % NW == wave) {
+        v4f x;
+        unsigned wo = wr[0];
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+          if (b / NW == i) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[r] = (float)(ad[i][r] + (double)c[i][r]);
+            wo = wr[i];
+          }
+        float* w = reinterpret_cast<float*>(Wc + 4 * k0 + wo);
+        float l[16];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) l[4 * q + j] = 4 * q + j < l16 ? -lb[q][j] : 0.f;
+        unit16<0>(x, l);
+        *reinterpret_cast<v4f*>(ub + l16 * PL + 4 * lk) = -x;
+        if (k0 + PB <= n) {
+          *reinterpret_cast<f4u*>(w) = x;
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (k0 + 4 * lk + r < n) w[r] = x[r];
+        }
+        if (b + NW < kb) load_lb(b + NW);
+      }
+      __syncthreads();
+      float u[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) u[j] = ub[(4 * lk + j) * PL + l16];
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        const int t = i * NW + wave;
+        if (t > b && t < nt) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) c[i] = mfma16x4(u[j], a[i][j], c[i]);
+          if (b + 1 < kb && t > b + 1)
+            a[i] = *reinterpret_cast<const f4u*>(Wc + 64 * (b + 1) + wr[i]);
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int t = i * NW + wave;
+      if (t >= kb && t < nt) {
+        v4f x;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[r] = (float)(ad[i][r] + (double)c[i][r]);
+        *reinterpret_cast<v4f*>(Pn + (16 * (t - kb) + l16) * PL + 4 * lk) = x;
+      }
+    }
+    __syncthreads();
+    if (wave == 0) {
+      const int R = n - k0;
+      int lane = thread_index(0);
+      float P[NS][PB];
+      unsigned em[NS];
+      int st[NS];
+#pragma unroll
+      for (int k = 0; k < NS; ++k) {
+        const int r = lane + 64 * k;
+        em[k] = r < R ? ~0u : 0u;
+        st[k] = -1;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const v4f x = *reinterpret_cast<const v4f*>(Pn + min(r, R - 1) * PL + 4 * q);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) P[k][4 * q + j] = x[j];
+        }
+      }
+      panel_cols_f32<NS, 0>(P, em, st, lane, pb);
+      lane = thread_index(0);
+      // the panel's rows to W, and the new order: the rows picked to the
+      // panel's positions, the rows they displace to the positions left
+      int* vac = reinterpret_cast<int*>(Pn);  // (read above by this wave only)
+      int left = 0, orig[NS];
+#pragma unroll
+      for (int k = 0; k < NS; ++k) orig[k] = perm[k0 + min(lane + 64 * k, R - 1)];
+#pragma unroll
+      for (int k = 0; k < NS; ++k) {
+        const int r = lane + 64 * k;
+        if (r < R) {
+          float* w = W + orig[k] * n + k0;
+          if (pb == PB) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              *reinterpret_cast<f4u*>(w + 4 * q) =
+                  f4u{P[k][4 * q], P[k][4 * q + 1], P[k][4 * q + 2], P[k][4 * q + 3]};
+          } else {
+#pragma unroll
+            for (int j = 0; j < PB; ++j)
+              if (j < pb) w[j] = P[k][j];
+          }
+        }
+        const bool gone = st[k] >= 0 && r >= pb;
+        const unsigned long long mb = __ballot(gone);
+        if (gone) vac[left + __popcll(mb & ((1ull << lane) - 1ull))] = r;
+        left += __popcll(mb);
+        if (st[k] >= 0) perm[k0 + st[k]] = orig[k];
+      }
+      asm volatile("" ::: "memory");  // a wave's LDS accesses execute in order
+      const bool out = lane < pb && st[0] < 0;
+      const unsigned long long mb = __ballot(out);
+      if (out) perm[k0 + vac[__popcll(mb & ((1ull << lane) - 1ull))]] = orig[0];
+    }
+    __syncthreads();
+  }
+}
 
 // R = B - A X in FP64 from the original A and the convergence test's norms,
 // NR (>= nrhs) columns: one row per thread, 8 columns of A per step, the
@@ -735,9 +990,8 @@ __device__ __forceinline__ void residual(const double* __restrict__ As,
 template <typename TF, int NT, int NMAX>
 // Occupancy: the kernel is latency-bound per system, so throughput follows
 // the systems in flight.  The 256-thread FP32 instances are held to 128
-// VGPRs (four workgroups per CU; 84 ms for 65,536 systems of sizes 16..256
-// against 110 ms at 160 VGPRs and 132 ms at 256), which they fit without
-// scratch once the loops rebuild the thread index (thread_index()).
+// VGPRs (four workgroups per CU), which they fit without scratch once the
+// loops rebuild the thread index (thread_index()).
 __global__ __launch_bounds__(NT, sizeof(TF) == 8 ? 1 : (NT == 256 ? 4 : (NT == 128 ? 1 : 2))) void lu_ir_batch_kernel(
     int count, int pos0, const int* __restrict__ list, const int* __restrict__ list_count,
     const int* __restrict__ order, const int64_t* __restrict__ wbase,
@@ -747,11 +1001,8 @@ __global__ __launch_bounds__(NT, sizeof(TF) == 8 ? 1 : (NT == 256 ? 4 : (NT == 1
     double* __restrict__ X, void* __restrict__ Wbase, int32_t* __restrict__ info,
     int32_t* __restrict__ iters, int* __restrict__ queue, int* __restrict__ queue_n) {
   constexpr int NW = NT / 64;
-  typedef typename Acc4<TF>::type AccT;
   __shared__ TF smem[LuSmem<TF, NMAX>::kWords];
-  __shared__ int piv[NMAX];
   __shared__ int perm[NMAX + 1];
-  __shared__ int s_tr[2 * PB], s_src[2 * PB], s_ntr;
   __shared__ double red_d[NW * (2 * kMaxRhs + 1)];
   __shared__ double s_bnorm[kMaxRhs];
   __shared__ int red_i[NW];
@@ -771,10 +1022,15 @@ __global__ __launch_bounds__(NT, sizeof(TF) == 8 ? 1 : (NT == 256 ? 4 : (NT == 1
     TF* __restrict__ W =
         static_cast<TF*>(Wbase) + wbase[n] + (int64_t)(pos - bstart[n]) * n * n;
 
+    if constexpr (sizeof(TF) == 4) {
+      factor_f32<NT, NMAX>(As, W, n, perm, smem, swave);
+    } else {
+    __shared__ int piv[NMAX];
+    __shared__ int s_tr[2 * PB], s_src[2 * PB], s_ntr;
     // ---- 1. W = A in row-major, TF (64 x 64 tiles through LDS, a tile's
     // loads all requested before its first store)
     {
-      constexpr int TS = NT >= 256 ? 64 : 32, PER = TS * TS / NT;
+      constexpr int TS = 64, PER = TS * TS / NT;
       TF* tile = smem;  // TS x (TS + 1)
       const int nt = (n + TS - 1) / TS;
       double v[PER];
@@ -890,7 +1146,7 @@ __global__ __launch_bounds__(NT, sizeof(TF) == 8 ? 1 : (NT == 256 ? 4 : (NT == 1
     // the panel area or (A_FROM_W, while wave 0 rewrites the panel area)
     // from W's panel columns; rows past the matrix only reach products that
     // are never stored.  B is -U12 from the U12 area.
-    constexpr int TB = sizeof(TF) == 8 ? 4 : (NMAX >= 128 ? 8 : 4);
+    constexpr int TB = 4;
     auto update_row = [&](auto a_from_w, int ti, int tj_begin, int tj_end, int k0, int T0,
                           int lane0) {
       const int lane = opaque(lane0), l16 = lane & 15, lk = lane >> 4;
@@ -905,59 +1161,14 @@ __global__ __launch_bounds__(NT, sizeof(TF) == 8 ? 1 : (NT == 256 ? 4 : (NT == 1
         for (int kk = 0; kk < PB / 4; ++kk)
           a[kk] = arow < n ? Pn[(arow - k0) * (PB + 1) + kk * 4 + lk] : TF(0);
       }
-      if constexpr (sizeof(TF) == 4) {
-        // FP32: the transposed tile C^T += (-U12)^T L21^T (the operands
-        // swapped), whose accumulator gives lane l row r0 + l % 16 and the
-        // four consecutive columns 4 (l / 16) .. of the tile: one 16-byte
-        // load and store per tile (rows past the matrix read its last row
-        // and are not stored)
-        const int row = r0 + l16;
-        TF* wr = W + min(row, n - 1) * n + T0 + 4 * lk;
-        for (int tj0 = tj_begin; tj0 < tj_end; tj0 += TB) {
-          AccT acc[TB];
-#pragma unroll
-          for (int j = 0; j < TB; ++j)
-            if (tj0 + j < tj_end) {
-              const int c0 = (tj0 + j) * 16;
-              if (T0 + c0 + 16 <= n) {
-                acc[j] = *reinterpret_cast<const f4u*>(wr + c0);
-              } else {
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                  acc[j][r] = T0 + c0 + 4 * lk + r < n ? wr[c0 + r] : TF(0);
-              }
-            }
-#pragma unroll
-          for (int j = 0; j < TB; ++j)
-            if (tj0 + j < tj_end) {
-              const int c0 = (tj0 + j) * 16;
-#pragma unroll
-              for (int kk = 0; kk < PB / 4; ++kk)
-                acc[j] = mfma16x4(Us[(kk * 4 + lk) * (NMAX + 1) + c0 + l16], a[kk], acc[j]);
-            }
-#pragma unroll
-          for (int j = 0; j < TB; ++j)
-            if (tj0 + j < tj_end && row < n) {
-              const int c0 = (tj0 + j) * 16;
-              if (T0 + c0 + 16 <= n) {
-                *reinterpret_cast<f4u*>(wr + c0) = acc[j];
-              } else {
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                  if (T0 + c0 + 4 * lk + r < n) wr[c0 + r] = acc[j][r];
-              }
-            }
-        }
-        return;
-      }
       for (int tj0 = tj_begin; tj0 < tj_end; tj0 += TB) {
-        AccT acc[TB];
+        v4d acc[TB];
 #pragma unroll
         for (int j = 0; j < TB; ++j) {
           const int col = T0 + (tj0 + j) * 16 + l16;
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const int row = r0 + acc_row<TF>(lane, r);
+            const int row = r0 + acc_row(lane, r);
             acc[j][r] = (tj0 + j < tj_end && row < n && col < n) ? W[row * n + col] : TF(0);
           }
         }
@@ -977,7 +1188,7 @@ __global__ __launch_bounds__(NT, sizeof(TF) == 8 ? 1 : (NT == 256 ? 4 : (NT == 1
           const int col = T0 + (tj0 + j) * 16 + l16;
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const int row = r0 + acc_row<TF>(lane, r);
+            const int row = r0 + acc_row(lane, r);
             if (tj0 + j < tj_end && row < n && col < n) W[row * n + col] = acc[j][r];
           }
         }
@@ -1070,31 +1281,23 @@ __global__ __launch_bounds__(NT, sizeof(TF) == 8 ? 1 : (NT == 256 ? 4 : (NT == 1
       const int tn = (nr + 15) / 16;
       const std::integral_constant<bool, false> from_lds;
       const std::integral_constant<bool, true> from_w;
-      if constexpr (NW == 1) {
-        // one wave: the whole update, then the next panel
-        for (int ti = 0; ti < tn; ++ti) update_row(from_lds, ti, 0, tn, k0, T0, lane);
+      // (a) tile column 0 (the next panel's columns) by every wave
+      for (int ti = wave; ti < tn; ti += NW) update_row(from_lds, ti, 0, 1, k0, T0, lane);
+      __syncthreads();
+      // (b) wave 0 factors the next panel and writes it out (panel area,
+      // W's columns T0 .., interchange lists); the others update tile
+      // columns 1.. with L21 from W
+      if (wave == 0) {
         TF P[NS][PB];
         int lg[NS];
         factor_panel(T0, P, lg, lane);
         write_panel(T0, P, lg, lane);
       } else {
-        // (a) tile column 0 (the next panel's columns) by every wave
-        for (int ti = wave; ti < tn; ti += NW) update_row(from_lds, ti, 0, 1, k0, T0, lane);
-        __syncthreads();
-        // (b) wave 0 factors the next panel and writes it out (panel area,
-        // W's columns T0 .., interchange lists); the others update tile
-        // columns 1.. with L21 from W
-        if (wave == 0) {
-          TF P[NS][PB];
-          int lg[NS];
-          factor_panel(T0, P, lg, lane);
-          write_panel(T0, P, lg, lane);
-        } else {
-          for (int ti = wave - 1; ti < tn; ti += NW - 1)
-            update_row(from_w, ti, 1, tn, k0, T0, lane);
-        }
+        for (int ti = wave - 1; ti < tn; ti += NW - 1)
+          update_row(from_w, ti, 1, tn, k0, T0, lane);
       }
       __syncthreads();
+    }
     }
 
     // ---- 3. solve and refine
@@ -1154,8 +1357,8 @@ __global__ __launch_bounds__(NT, sizeof(TF) == 8 ? 1 : (NT == 256 ? 4 : (NT == 1
       auto solve = [&](auto nr) {
         constexpr int NR = decltype(nr)::value;
         if constexpr (sizeof(TF) == 4) {
-          tri_solve_f32<NT, true, NR>(W, n, y, diag, tid);
-          tri_solve_f32<NT, false, NR>(W, n, y, diag, tid);
+          tri_solve_f32<NT, true, NR>(W, n, perm, y, diag, tid);
+          tri_solve_f32<NT, false, NR>(W, n, perm, y, diag, tid);
         } else {
           tri_solve<TF, NT, true, NR>(W, n, y, diag, tid);
           tri_solve<TF, NT, false, NR>(W, n, y, diag, tid);
@@ -1197,7 +1400,8 @@ __global__ __launch_bounds__(NT, sizeof(TF) == 8 ? 1 : (NT == 256 ? 4 : (NT == 1
       else
         residual<TF, NT, kMaxRhs>(As, Bs, n, nrhs, xs, rv, tid, lane, wave, red_d, s_bnorm,
                                   it == 0, anorm, worst, bad);
-      if (!bad) { converged = 1; break; }
+      converged = !bad;
+      if (converged && (kRefactor || worst <= kDone)) break;
       // stop on the iteration limit, or when a step gains less than 2x
       if (it >= kMaxIter || !(worst < 0.5 * prev)) break;
       prev = worst;
@@ -1227,17 +1431,18 @@ typedef void (*LuKernel)(int, int, const int*, const int*, const int*, const int
 // LDS is sized for the largest system of a launch: 64, 128 or 256
 int nmax_for(int n) { return n <= 64 ? 64 : (n <= 128 ? 128 : 256); }
 
-template <int NMAX>
-LuKernel lu_kernel_nt(int nt) {
-  if (nt == 64) return lu_ir_batch_kernel<float, 64, NMAX>;
-  if (nt == 128) return lu_ir_batch_kernel<float, 128, NMAX>;
-  return lu_ir_batch_kernel<float, 256, NMAX>;
-}
-
+// At most four 16-row tiles per wave (they live in registers): a wave up to 64
+// rows, two up to 128, four above.  Fewer waves with eight or sixteen tiles
+// would need over half of a SIMD's registers each.
 LuKernel lu_kernel_for(int nt, int nmax) {
-  if (nmax == 64) return lu_kernel_nt<64>(nt);
-  if (nmax == 128) return lu_kernel_nt<128>(nt);
-  return lu_kernel_nt<256>(nt);
+  if (nmax == 64) {
+    if (nt == 64) return lu_ir_batch_kernel<float, 64, 64>;
+    if (nt == 128) return lu_ir_batch_kernel<float, 128, 64>;
+    return lu_ir_batch_kernel<float, 256, 64>;
+  }
+  if (nmax == 128)
+    return nt == 256 ? lu_ir_batch_kernel<float, 256, 128> : lu_ir_batch_kernel<float, 128, 128>;
+  return lu_ir_batch_kernel<float, 256, 256>;
 }
 
 int lu_default_threads(int n) { return n <= 48 ? 64 : (n <= 128 ? 128 : 256); }
@@ -1308,6 +1513,7 @@ int lu_autotune(eamd_handle* h, int n, int nrhs) {
       (void)hipEventCreate(&e1);
       float best_ms = 1e30f;
       for (int nt : {64, 128, 256}) {
+        if (nt < nmax_for(N)) continue;
         LuKernel k = lu_kernel_for(nt, nmax_for(N));
         float ms_min = 1e30f;
         for (int rep = 0; rep < 2; ++rep) {
