@@ -81,21 +81,23 @@ __global__ __launch_bounds__(256) void trinv64_kernel(int n, const double* __res
   __syncthreads();
   const int ti = (wave & 1) * 16, tj = (wave >> 1) * 16;
   {
-    v4d acc = {0.0, 0.0, 0.0, 0.0};
+    v4d a[4] = {};
 #pragma unroll
     for (int k = 0; k < 32; k += 4)
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(S[(32 + ti + l16) * LD + k + lk],
-                                                 X[(k + lk) * LD + tj + l16], acc, 0, 0, 0);
+      a[k / 8] = __builtin_amdgcn_mfma_f64_16x16x4f64(S[(32 + ti + l16) * LD + k + lk],
+                                                      X[(k + lk) * LD + tj + l16], a[k / 8], 0, 0, 0);
+    const v4d acc = (a[0] + a[1]) + (a[2] + a[3]);
 #pragma unroll
     for (int r = 0; r < 4; ++r) Y[(ti + lk + 4 * r) * 33 + tj + l16] = acc[r];
   }
   __syncthreads();
   {
-    v4d acc = {0.0, 0.0, 0.0, 0.0};
+    v4d a[4] = {};
 #pragma unroll
     for (int k = 0; k < 32; k += 4)
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-X[(32 + ti + l16) * LD + 32 + k + lk],
-                                                 Y[(k + lk) * 33 + tj + l16], acc, 0, 0, 0);
+      a[k / 8] = __builtin_amdgcn_mfma_f64_16x16x4f64(-X[(32 + ti + l16) * LD + 32 + k + lk],
+                                                      Y[(k + lk) * 33 + tj + l16], a[k / 8], 0, 0, 0);
+    const v4d acc = (a[0] + a[1]) + (a[2] + a[3]);
 #pragma unroll
     for (int r = 0; r < 4; ++r) X[(32 + ti + lk + 4 * r) * LD + tj + l16] = acc[r];
   }
@@ -172,6 +174,20 @@ __global__ __launch_bounds__(256) void trsm_block_kernel(int n, const double* __
       }
     }
   };
+  // 16 rows of a 64 x 64 block times 64 rows of X or Y: four sums of 16
+  // products each, so that a result carries the rounding of short sums (one
+  // chain of 32 products in each of two sums: 1.40e-16 off exact results at
+  // n = 200 .. 700, and 1.29e-16 so) and a product waits for every fourth
+  auto product = [&](const double (&m)[SB / 4], const double* xb) {
+    v4d a[4] = {};
+#pragma unroll
+    for (int u = 0; u < SB / 16; ++u)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        a[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(m[u * 4 + j], xb[(u * 16 + j) * XLD], a[j], 0,
+                                                    0, 0);
+    return (a[0] + a[1]) + (a[2] + a[3]);
+  };
   load_t(0);
   __syncthreads();
 #pragma unroll
@@ -189,44 +205,24 @@ __global__ __launch_bounds__(256) void trsm_block_kernel(int n, const double* __
         di[u * 4 + j] = w.x;
         di[u * 4 + j + 1] = w.y;
       }
-    v4d a0 = {0.0, 0.0, 0.0, 0.0}, a1 = {0.0, 0.0, 0.0, 0.0};
+    v4d acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int e = 0; e < NSUB - 1; ++e) {
       if (e >= d) break;
-      const double* xb = Xs + (sub(e) * SB + lk * 4) * XLD + l16;
-#pragma unroll
-      for (int u = 0; u < SB / 16; ++u)
-#pragma unroll
-        for (int j = 0; j < 4; j += 2) {
-          a0 = __builtin_amdgcn_mfma_f64_16x16x4f64(t[e][u * 4 + j], xb[(u * 16 + j) * XLD], a0, 0,
-                                                    0, 0);
-          a1 = __builtin_amdgcn_mfma_f64_16x16x4f64(t[e][u * 4 + j + 1],
-                                                    xb[(u * 16 + j + 1) * XLD], a1, 0, 0, 0);
-        }
+      acc += product(t[e], Xs + (sub(e) * SB + lk * 4) * XLD + l16);
     }
     if (d + 1 < NSUB && d + 1 < nsub) load_t(d + 1);
     // lane (lk, l16) register r: row lk + 4 r, column l16 of the wave's tile
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int row = wave * 16 + lk + 4 * r;
-      const double y = Xs[(rb + row) * XLD + l16] - (a0[r] + a1[r]);
+      const double y = Xs[(rb + row) * XLD + l16] - acc[r];
       Ys[row * XLD + l16] = rb + row < rows ? y : 0.0;
     }
     __syncthreads();
-    v4d x0 = {0.0, 0.0, 0.0, 0.0}, x1 = {0.0, 0.0, 0.0, 0.0};
-    const double* yb = Ys + lk * 4 * XLD + l16;
+    const v4d x = product(di, Ys + lk * 4 * XLD + l16);
 #pragma unroll
-    for (int u = 0; u < SB / 16; ++u)
-#pragma unroll
-      for (int j = 0; j < 4; j += 2) {
-        x0 = __builtin_amdgcn_mfma_f64_16x16x4f64(di[u * 4 + j], yb[(u * 16 + j) * XLD], x0, 0, 0,
-                                                  0);
-        x1 = __builtin_amdgcn_mfma_f64_16x16x4f64(di[u * 4 + j + 1], yb[(u * 16 + j + 1) * XLD],
-                                                  x1, 0, 0, 0);
-      }
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      Xs[(rb + wave * 16 + lk + 4 * r) * XLD + l16] = x0[r] + x1[r];
+    for (int r = 0; r < 4; ++r) Xs[(rb + wave * 16 + lk + 4 * r) * XLD + l16] = x[r];
     __syncthreads();
   }
   double* xp = X + (int64_t)c0 * ldx + r0 + tid;
