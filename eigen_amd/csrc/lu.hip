@@ -73,8 +73,163 @@ __global__ __launch_bounds__(256) void laswp_perm_kernel(T* __restrict__ W, int6
     if (ok) W[(int64_t)(r0 + s_pos[s2]) * ldw + c] = buf[s_src[s2] * CW + tc];
 }
 
+typedef double v2du __attribute__((ext_vector_type(2), aligned(8)));
+
+// x[r] += (lane T of each row of sixteen of x[r]) * l[T] for T = 0 .. 14: the
+// unit lower solve of 16 rows (lane l16: row l16, l = minus its strict lower
+// part), four columns in registers.  The wait states cover the VALU write just
+// before.
+template <int T>
+__device__ __forceinline__ void unit16(double (&x)[4], const double (&l)[16]) {
+  if constexpr (T < 15) {
+    asm volatile("s_nop 1\n\tv_fmac_f64_dpp %0, %0, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %1, %1, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %2, %2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %3, %3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+                 : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3])
+                 : "v"(l[T]), "n"(T));
+    unit16<T + 1>(x, l);
+  }
+}
+
+// X <- L^{-1} X in FP64 (L unit lower nb x nb, nb <= 16 MAXB; both row-major):
+// sixteen columns of X per wave, all in registers as 16 x 16 tiles (lane (l16,
+// lk): row l16, columns 4 lk .. + 3), and no wave waits for another.  Per
+// 16-row block: the solve against L's diagonal block by the FMA's lane
+// broadcast, the solved rows through LDS into the other operand's layout, and
+// four products for every tile below, L's values for them requested before
+// the solve.  What bounds it: the blocks' chain (a solve and an LDS round
+// trip), and with many columns the products.  32 rows: 12.5 us with a thread
+// per column and 32 dependent rows from LDS, 4.5 so; 256 rows x up to 16128
+// columns: 136 us on average then, 75 now.
+template <int MAXB>
+__global__ __launch_bounds__(256) void trsm_llu64_kernel(const double* __restrict__ L, int64_t ldl,
+                                                         int nb, double* __restrict__ X,
+                                                         int64_t ldx, int ncols) {
+  constexpr int P = 18;  // LDS row stride
+  __shared__ __align__(16) double s_u[4][16 * P];
+  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, lk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c0 = (blockIdx.x * 4 + wave) * 16;
+  if (c0 >= ncols) return;
+  double* ub = s_u[wave];
+  const int nblk = (nb + 15) / 16, col = c0 + 4 * lk;
+  const bool whole = c0 + 16 <= ncols;
+  // operand row m of a product stands for column 4 (m % 4) + m / 4, so that a
+  // lane's four results are four consecutive columns
+  const int sig = 4 * (l16 & 3) + (l16 >> 2);
+  v4d x[MAXB];
+#pragma unroll
+  for (int i = 0; i < MAXB; ++i) {
+    x[i] = v4d{0.0, 0.0, 0.0, 0.0};  // (rows past nb stay zero)
+    const int row = 16 * i + l16;
+    if (row < nb) {
+      const double* p = X + (int64_t)row * ldx;
+      if (whole) {
+        const v2du a = *reinterpret_cast<const v2du*>(p + col);
+        const v2du b = *reinterpret_cast<const v2du*>(p + col + 2);
+        x[i] = v4d{a.x, a.y, b.x, b.y};
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[i][r] = p[min(col + r, ncols - 1)];
+      }
+    }
+  }
+  // the next diagonal block's row, requested a block ahead
+  double d[16];
+  auto load_diag = [&](int b) {
+    const double* p = L + (int64_t)min(16 * b + l16, nb - 1) * ldl + 16 * b;
+    if (16 * b + 16 <= nb) {
+#pragma unroll
+      for (int k = 0; k < 16; k += 2) {
+        const v2du a = *reinterpret_cast<const v2du*>(p + k);
+        d[k] = a.x;
+        d[k + 1] = a.y;
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) d[k] = p[min(k, nb - 1 - 16 * b)];
+    }
+  };
+  load_diag(0);
+#pragma unroll 1
+  for (int b = 0; b < nblk; ++b) {
+    // L: the diagonal block's row (minus its strict lower part) and the tiles
+    // below, lane (l16, lk): row l16, columns 4 lk .. + 3; rows past nb repeat
+    // the last one (their results are not kept)
+    double l[16], t[MAXB][4];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) l[k] = k < l16 && 16 * b + l16 < nb ? -d[k] : 0.0;
+#pragma unroll
+    for (int i = 1; i < MAXB; ++i)
+      if (i > b && i < nblk) {  // (block b is whole)
+        const double* p = L + (int64_t)min(16 * i + l16, nb - 1) * ldl + 16 * b + 4 * lk;
+        const v2du a = *reinterpret_cast<const v2du*>(p);
+        const v2du c = *reinterpret_cast<const v2du*>(p + 2);
+        t[i][0] = a.x;
+        t[i][1] = a.y;
+        t[i][2] = c.x;
+        t[i][3] = c.y;
+      }
+    if (b + 1 < nblk) load_diag(b + 1);
+    double y[4], y0[4];
+#pragma unroll
+    for (int i = 0; i < MAXB; ++i)
+      if (i == b) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) y[r] = x[i][r];
+      }
+    // a product's result needs these wait states before inline assembly may
+    // read it (the compiler does not look into it)
+    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" : "+v"(y[0]), "+v"(y[1]), "+v"(y[2]), "+v"(y[3]));
+#pragma unroll
+    for (int r = 0; r < 4; ++r) y0[r] = y[r];
+    unit16<0>(y, l);
+    // the broadcast adds zero times the solved value to the rows above it,
+    // which an infinity or a NaN would spoil: such a block again, masked
+    const double sum = (y[0] - y[0]) + (y[1] - y[1]) + ((y[2] - y[2]) + (y[3] - y[3]));
+    if (__ballot(!(sum == 0.0))) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) y[r] = y0[r];
+#pragma unroll
+      for (int k = 0; k < 15; ++k)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const double z = __shfl(y[r], (lane & 48) + k);
+          y[r] = l16 > k && 16 * b + l16 < nb ? fma(l[k], z, y[r]) : y[r];
+        }
+    }
+    if (16 * b + l16 < nb) {
+      double* p = X + (int64_t)(16 * b + l16) * ldx;
+      if (whole) {
+        *reinterpret_cast<v2du*>(p + col) = v2du{y[0], y[1]};
+        *reinterpret_cast<v2du*>(p + col + 2) = v2du{y[2], y[3]};
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (col + r < ncols) p[col + r] = y[r];
+      }
+    }
+    if (b + 1 == nblk) break;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) ub[l16 * P + 4 * lk + r] = -y[r];
+    asm volatile("" ::: "memory");  // a wave's LDS accesses execute in order
+    double u[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) u[j] = ub[(4 * lk + j) * P + sig];
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int i = 1; i < MAXB; ++i)
+      if (i > b && i < nblk) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          x[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(u[j], t[i][j], x[i], 0, 0, 0);
+      }
+  }
+}
+
 // X <- L^{-1} X, L unit lower nb x nb (row-major, ld ldl), X nb x ncols
-// (row-major).  One workgroup per CB columns, the X block resident in LDS.
+// (row-major), in FP32.  One workgroup per CB columns, the X block resident in LDS.
 // Per 32-row diagonal block: one thread per column solves the block from
 // registers (compile-time indices, L broadcast from LDS, no barrier inside),
 // then all threads update the rows below with 32-long dot products.
@@ -319,19 +474,36 @@ template <typename T>
 int trsm_llu_rowmajor(hipStream_t s, const T* L, int64_t ldl, int nb, T* X, int64_t ldx,
                       int ncols) {
   if (ncols <= 0 || nb <= 0) return kOk;
-  constexpr int CB = 32;
-  size_t lds = sizeof(T) * (size_t)((nb + 31) & ~31) * (CB + 1);
-  auto kern = trsm_llu_kernel<T, CB>;
-  static bool attr_set = false;
-  if (!attr_set) {
-    EAMD_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 150 * 1024));
-    attr_set = true;
+  if constexpr (sizeof(T) == 8) {
+    if (nb > 256) {
+      set_error("trsm_llu: panel width %d > 256", nb);
+      return kErrUnsupported;
+    }
+    const dim3 grid(ceil_div(ncols, 64));
+#define EAMD_LLU(MAXB)                                                                        \
+  hipLaunchKernelGGL(trsm_llu64_kernel<MAXB>, grid, dim3(256), 0, s, L, ldl, nb, X, ldx, ncols)
+    if (nb <= 32) EAMD_LLU(2);
+    else if (nb <= 64) EAMD_LLU(4);
+    else if (nb <= 128) EAMD_LLU(8);
+    else EAMD_LLU(16);
+#undef EAMD_LLU
+    EAMD_HIP(hipGetLastError());
+    return kOk;
+  } else {
+    constexpr int CB = 32;
+    size_t lds = sizeof(T) * (size_t)((nb + 31) & ~31) * (CB + 1);
+    auto kern = trsm_llu_kernel<T, CB>;
+    static bool attr_set = false;
+    if (!attr_set) {
+      EAMD_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   150 * 1024));
+      attr_set = true;
+    }
+    hipLaunchKernelGGL(kern, dim3(ceil_div(ncols, CB)), dim3(256), lds, s, L, ldl, nb, X, ldx,
+                       ncols);
+    EAMD_HIP(hipGetLastError());
+    return kOk;
   }
-  hipLaunchKernelGGL(kern, dim3(ceil_div(ncols, CB)), dim3(256), lds, s, L, ldl, nb, X, ldx,
-                     ncols);
-  EAMD_HIP(hipGetLastError());
-  return kOk;
 }
 
 // The panel's row permutation on ncols columns starting at X (row 0 = the
