@@ -578,38 +578,6 @@ constexpr int kLeaf64MaxG = 16;  // 16384 rows
 typedef double v2du __attribute__((ext_vector_type(2), aligned(8)));
 typedef double v2d __attribute__((ext_vector_type(2)));
 
-// a[C + q] += (lane (C + q) % 16 of each row of sixteen of u) * l for q = Q0
-// .. 7.  The wait states cover a VALU write of u just before (a DPP operand
-// needs two); they cost as much as an FMA, so one wait serves eight.
-template <int C, int Q0>
-__device__ __forceinline__ void fmac_bcast8(double (&a)[LW], double u, double l) {
-#define EAMD_FM(I, N) "v_fmac_f64_dpp %" #I ", %8, %9 row_newbcast:%" #N " row_mask:0xf bank_mask:0xf\n\t"
-  constexpr int N0 = C & 15;
-  if constexpr (Q0 == 0) {
-    asm volatile("s_nop 1\n\t" EAMD_FM(0, 10) EAMD_FM(1, 11) EAMD_FM(2, 12) EAMD_FM(3, 13)
-                     EAMD_FM(4, 14) EAMD_FM(5, 15) EAMD_FM(6, 16) EAMD_FM(7, 17)
-                 : "+v"(a[C]), "+v"(a[C + 1]), "+v"(a[C + 2]), "+v"(a[C + 3]), "+v"(a[C + 4]),
-                   "+v"(a[C + 5]), "+v"(a[C + 6]), "+v"(a[C + 7])
-                 : "v"(u), "v"(l), "n"(N0), "n"(N0 + 1), "n"(N0 + 2), "n"(N0 + 3), "n"(N0 + 4),
-                   "n"(N0 + 5), "n"(N0 + 6), "n"(N0 + 7));
-  } else {
-    // the current group's later columns: two at a time
-#define EAMD_F2(Q)                                                                              \
-  if constexpr (Q >= Q0)                                                                        \
-    asm volatile("s_nop 1\n\tv_fmac_f64_dpp %0, %2, %3 row_newbcast:%4 row_mask:0xf bank_mask:0xf\n\t" \
-                 "v_fmac_f64_dpp %1, %2, %3 row_newbcast:%5 row_mask:0xf bank_mask:0xf"        \
-                 : "+v"(a[C + Q]), "+v"(a[C + Q + 1])                                           \
-                 : "v"(u), "v"(l), "n"(N0 + Q), "n"(N0 + Q + 1));                               \
-  else if constexpr (Q + 1 >= Q0)                                                               \
-    asm volatile("s_nop 1\n\tv_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" \
-                 : "+v"(a[C + Q + 1])                                                           \
-                 : "v"(u), "v"(l), "n"(N0 + Q + 1));
-    EAMD_F2(0) EAMD_F2(2) EAMD_F2(4) EAMD_F2(6)
-#undef EAMD_F2
-  }
-#undef EAMD_FM
-}
-
 // Maximum over the lanes of each row of sixteen (all of them get it).
 __device__ __forceinline__ unsigned row_max_u32(unsigned k) {
   k = max(k, (unsigned)__builtin_amdgcn_mov_dpp((int)k, 0xB1, 0xf, 0xf, false));

@@ -43,6 +43,35 @@ __device__ __forceinline__ double readlane_f64(double x, int l) {
                               (unsigned)__builtin_amdgcn_readlane((int)bits, l));
 }
 
+// x of rows 0..15 of each half wave (lanes 0..15 and 32..47), in both of its
+// rows of sixteen.
+__device__ __forceinline__ double low_rows(double x) {
+  const long long b = __double_as_longlong(x);
+  const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
+  const auto l2 = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+  const auto h2 = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+  return __longlong_as_double(((long long)h2[0] << 32) | l2[0]);
+}
+
+// a[j] += (lane j % 16 of each row of sixteen of lo for j < 16, of hi above) *
+// l for j = FROM .. 31.
+template <int FROM>
+__device__ __forceinline__ void fmac_bcast_from(double (&a)[32], double lo, double hi, double l) {
+  if constexpr (FROM < 8) fmac_bcast8<0, FROM>(a, lo, l);
+  if constexpr (FROM < 16) fmac_bcast8<8, (FROM > 8 ? FROM - 8 : 0)>(a, lo, l);
+  if constexpr (FROM < 24) fmac_bcast8<16, (FROM > 16 ? FROM - 16 : 0)>(a, hi, l);
+  if constexpr (FROM < 32) fmac_bcast8<24, (FROM > 24 ? FROM - 24 : 0)>(a, hi, l);
+}
+
+// f(integral_constant<int, i>) for i = I .. 31, unrolled
+template <int I = 0, typename F>
+__device__ __forceinline__ void each32(F&& f) {
+  if constexpr (I < 32) {
+    f(std::integral_constant<int, I>{});
+    each32<I + 1>(f);
+  }
+}
+
 // One 16 x 16 f64 MFMA tile product over LDS operands, accumulated into
 // acc: lane (lk = lane / 16, l16 = lane % 16) supplies F(l16, k) and
 // G(k, l16) for k = 4 q + lk, and register r of acc holds D(lk + 4 r, l16)
@@ -64,10 +93,15 @@ __device__ __forceinline__ void tile16(v4d& acc, int kdim, int l16, int lk, FF F
 // LDS and also form L^-1 there; L goes back to A, L^-1 (bsp x bsp, zero
 // above the diagonal, identity on the padding) to Li (column-major, ld
 // kMaxNb).  Factorization in 32-column sub-blocks: wave 0 factors the 32 x 32
-// diagonal sub-block with one row per lane in registers (each column is
-// broadcast through LDS, one division per column: the column is scaled by
-// 1 / L_cc), one thread per row below solves against it, and the trailing
-// lower part takes the rank-32 update as 16 x 16 MFMA tiles.  The inverse:
+// diagonal sub-block with one row per lane in registers (a column's values
+// reach the others by the FMA's own lane broadcast; one division per column:
+// the column is scaled by 1 / L_cc), one thread per row below solves against
+// it the same way, and the trailing lower part takes the rank-32 update as
+// 16 x 16 MFMA tiles.  With two readlanes per FMA in the sub-block and an LDS
+// read per FMA in the rows below and in the diagonal blocks' inverses, a
+// 128-block took 98 us, 80 now: the 32-column chains (a square root, a
+// reciprocal and an FMA's turn each, 500 cycles a column) are two fifths of
+// it.  The inverse:
 // the four 32 x 32 diagonal blocks are inverted by one wave each (lane j
 // forms column j), then block row i of L^-1 is X_ij = -X_ii (sum over
 // k = j..i-1 of L_ik X_kj), block rows in order, each product on MFMA.
@@ -114,22 +148,25 @@ __global__ __launch_bounds__(256) void potf2_inv_kernel(double* __restrict__ A, 
       int f = -1;
       double myr = 0.0;  // 1 / L_cc of this lane's row c = li
       double diag = readlane_f64(x[0], 0);
-#pragma unroll
-      for (int c = 0; c < 32; ++c) {
+      each32([&](auto cc) __attribute__((always_inline)) {
+        constexpr int c = decltype(cc)::value;
         f = (f < 0 && diag <= 0.0) ? c : f;
         const double d = sqrt(diag), r = recip(d);
         x[c] = li == c ? d : (li > c ? x[c] * r : x[c]);
         myr = li == c ? r : myr;
-        if (c < 31) {
+        if constexpr (c < 31) {
           // the next column first (its diagonal is the next step's input),
-          // then the rest of the rank-1 update, column c read lane by lane
-          // (lanes above the diagonal carry values that are never stored)
+          // then the rest of the rank-1 update, column c by the FMA's lane
+          // broadcast (lanes above the diagonal carry values that are never
+          // stored)
           x[c + 1] -= x[c] * readlane_f64(x[c], c + 1);
           diag = readlane_f64(x[c + 1], c + 1);
-#pragma unroll
-          for (int j = c + 2; j < 32; ++j) x[j] -= x[c] * readlane_f64(x[c], j);
+          if constexpr (c < 30) {
+            const double lo = c < 14 ? low_rows(x[c]) : 0.0;
+            fmac_bcast_from<c + 2>(x, lo, x[c], -x[c]);
+          }
         }
-      }
+      });
       if (lane < 32) {
         s_dinv[kb + li] = myr;
 #pragma unroll
@@ -147,24 +184,14 @@ __global__ __launch_bounds__(256) void potf2_inv_kernel(double* __restrict__ A, 
       double y[32];
 #pragma unroll
       for (int c = 0; c < 32; ++c) y[c] = Sx(i, kb + c);
-      // row c of L is read one step ahead (the LDS reads of a step are in
-      // flight while the previous step computes); four partial sums, the
-      // newest term (q = c - 1) last, so only it waits for y[c - 1]
-      double lr[2][32];
-#pragma unroll
-      for (int c = 0; c < 32; ++c) {
-        if (c == 0) {
-#pragma unroll
-          for (int q = 0; q < 1; ++q) lr[1][q] = Sx(kb + 1, kb + q);
-        } else if (c < 31) {
-#pragma unroll
-          for (int q = 0; q <= c; ++q) lr[(c + 1) & 1][q] = Sx(kb + c + 1, kb + q);
-        }
-        double v[4] = {y[c], 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int q = 0; q < c; ++q) v[(c - 1 - q) & 3] -= y[q] * lr[c & 1][q];
-        y[c] = ((v[0] + v[1]) + (v[2] + v[3])) * s_dinv[kb + c];
-      }
+      // right-looking along the row: column q of L is read once, an element
+      // per lane, and broadcast by the FMA (an LDS read per FMA before)
+      each32([&](auto qq) __attribute__((always_inline)) {
+        constexpr int q = decltype(qq)::value;
+        y[q] *= s_dinv[kb + q];
+        if constexpr (q < 31)
+          fmac_bcast_from<q + 1>(y, Sx(kb + l16, kb + q), Sx(kb + 16 + l16, kb + q), -y[q]);
+      });
 #pragma unroll
       for (int c = 0; c < 32; ++c) Sx(i, kb + c) = y[c];
     }
@@ -209,16 +236,13 @@ __global__ __launch_bounds__(256) void potf2_inv_kernel(double* __restrict__ A, 
     const int b0 = wave * 32, j = lane & 31;
     double x[32];
 #pragma unroll
-    for (int i = 0; i < 32; ++i) {
-      double sp[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int k = 0; k < i; ++k) sp[(i - 1 - k) & 3] += Sx(b0 + i, b0 + k) * x[k];
-      const double sacc = (sp[0] + sp[1]) + (sp[2] + sp[3]);
-      const double di = s_dinv[b0 + i];
-      x[i] = i < j ? 0.0 : (i == j ? di : -sacc * di);
-      // keeps the next row's LDS reads from being hoisted (register bound)
-      asm volatile("" ::: "memory");
-    }
+    for (int i = 0; i < 32; ++i) x[i] = i == j ? 1.0 : 0.0;
+    each32([&](auto kk) __attribute__((always_inline)) {
+      constexpr int k = decltype(kk)::value;
+      x[k] = k < j ? 0.0 : x[k] * s_dinv[b0 + k];
+      if constexpr (k < 31)
+        fmac_bcast_from<k + 1>(x, Sx(b0 + l16, b0 + k), Sx(b0 + 16 + l16, b0 + k), -x[k]);
+    });
     asm volatile("" ::: "memory");
     if (lane < 32) {
 #pragma unroll
