@@ -736,16 +736,16 @@ __device__ void rank_update_wave(int64_t s, const int64_t* __restrict__ offL,
 }
 
 __global__ __launch_bounds__(256) void llt_rank_update_kernel(
-    int64_t count, int spans, const int64_t* __restrict__ offL, const int32_t* __restrict__ nv,
+    int64_t count, int many, int all, const int64_t* __restrict__ offL, const int32_t* __restrict__ nv,
     double* __restrict__ Lall, const int64_t* __restrict__ offv, const double* __restrict__ V,
     const double* __restrict__ sigmas, int upper, int32_t* __restrict__ info) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int64_t span0 = spans ? (int64_t)blockIdx.x * kRankSpan
-                              : (int64_t)(blockIdx.x / 8) * kRankSpan;
+  const unsigned per = 8u / many;  // workgroups of a span
+  const int64_t span0 = (int64_t)(blockIdx.x / per) * kRankSpan;
   int size;
-  if (rank_span_small(span0, count, nv, lane, size)) return;
-  const int first = spans ? 8 * wave : 4 * (int)(blockIdx.x % 8) + wave, many = spans ? 8 : 1;
+  if (!all && rank_span_small(span0, count, nv, lane, size)) return;
+  const int first = (4 * (int)(blockIdx.x % per) + wave) * many;
   for (int q = 0; q < many; ++q) {
     const int64_t s = span0 + first + q;
     if (s < count) rank_update_wave(s, offL, nv, Lall, offv, V, sigmas, upper, info);
@@ -762,13 +762,20 @@ int llt_rank_update_batched(eamd_handle* h, int64_t count, const int64_t* offL, 
     set_error("rank update: %lld systems exceed one launch", (long long)count);
     return kErrUnsupported;
   }
-  hipLaunchKernelGGL(llt_rank_update_small_kernel, dim3((unsigned)nspan), dim3(256), 0, h->stream,
-                     count, offL, n, L, offv, v, sigma, upper, info);
-  // with 2048 spans a wave for every eight factors still fills the chip
-  const int spans = nspan >= 2048 ? 1 : 0;
-  hipLaunchKernelGGL(llt_rank_update_kernel, dim3((unsigned)(spans ? nspan : 8 * nspan)),
-                     dim3(256), 0, h->stream, count, spans, offL, n, L, offv, v, sigma, upper,
-                     info);
+  // below 4096 factors the one launch of a wave each: a second launch, 4 us,
+  // would cost larger factors more (2735 of 35 and 51: 139 against 146 us)
+  // than eight lanes gain on small ones (1853 of 21: 57 against 49)
+  const int all = nspan < 128;
+  if (!all)
+    hipLaunchKernelGGL(llt_rank_update_small_kernel, dim3((unsigned)nspan), dim3(256), 0,
+                       h->stream, count, offL, n, L, offv, v, sigma, upper, info);
+  // one to eight factors per wave: few enough that 64 Ki waves, a dozen turns
+  // of the chip, remain (99792 factors of 7 and 69: eight a wave left two and
+  // a half turns, 1.87 ms against 1.54), and few workgroups that find only
+  // small factors (a million of up to 32: 250 Ki of them with one a wave)
+  const int many = nspan >= 16384 ? 8 : (nspan >= 8192 ? 4 : (nspan >= 4096 ? 2 : 1));
+  hipLaunchKernelGGL(llt_rank_update_kernel, dim3((unsigned)(8 / many * nspan)), dim3(256), 0,
+                     h->stream, count, many, all, offL, n, L, offv, v, sigma, upper, info);
   EAMD_HIP(hipGetLastError());
   return kOk;
 }

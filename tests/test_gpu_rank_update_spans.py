@@ -67,3 +67,37 @@ def test_sizes(sizes, upper):
 @pytest.mark.parametrize("n", [2, 9, 24, 32, 50])
 def test_failed_downdate_beside_others(n):
     run([n] * 20, np.where(np.arange(20) % 4 == 3, 0.5, -0.01), False, fail=(2, 17))
+
+
+@pytest.mark.parametrize("copies", [64, 2100, 4200, 8300])
+@pytest.mark.parametrize("base", [[0, 1, 7, 8, 9, 15, 16, 17, 23, 24, 25, 31, 32, 2, 5, 12] * 4,
+                                  [3, 1, 2, 33, 5, 2, 9, 40] * 4 + [2, 4, 32, 1] * 8])
+def test_counts_that_change_the_launches(base, copies):
+    """64 factors, repeated: from 4096 factors on small spans take eight lanes
+    per factor, and the other spans one, two, four or eight factors a wave.
+    Every copy must come out alike, and the first as the oracle's update."""
+    from eigen_amd import batched
+    real = np.asarray(base, dtype=np.int64)
+    nL, nV = int((real ** 2).sum()), int(real.sum())
+    o1 = np.concatenate([[0], np.cumsum(real ** 2)[:-1]])
+    o2 = np.concatenate([[0], np.cumsum(real)[:-1]])
+    L, V = np.zeros(nL), np.random.default_rng(4).standard_normal(nV)
+    for i, n in enumerate(real):
+        if n:
+            L[o1[i]:o1[i] + n * n] = np.linalg.cholesky(inputs.spd(9100 + i, int(n))).flatten("F")
+    sig = np.where(np.arange(64) % 3 == 1, -0.01, 1.5)
+    rep = torch.arange(copies, device="cuda")[:, None]
+    t = lambda a: torch.tensor(a, device="cuda")
+    Ld = t(L).repeat(copies)
+    info = batched.llt_rank_update_batched(
+        (rep * nL + t(o1)).reshape(-1), t(real.astype(np.int32)).repeat(copies), Ld,
+        (rep * nV + t(o2)).reshape(-1), t(V).repeat(copies), t(sig).repeat(copies))
+    out = Ld.reshape(copies, nL)
+    assert bool((info == -1).all()) and bool((out == out[0]).all())
+    got = out[0].cpu().numpy()
+    for i, n in enumerate(real):
+        l0 = L[o1[i]:o1[i] + n * n].reshape(n, n, order="F")
+        ref, _ = po.llt_rank_update(np.asfortranarray(l0), V[o2[i]:o2[i] + n], sig[i])
+        tol = 64 * max(n, 1) * EPS * 2 * np.sqrt(2 * max(n, 1))
+        g = got[o1[i]:o1[i] + n * n].reshape(n, n, order="F")
+        assert np.all(np.abs(np.tril(g) - np.tril(ref)) <= tol), (i, n)
