@@ -296,132 +296,160 @@ __global__ __launch_bounds__(256) void trsm_llu_kernel(const T* __restrict__ L, 
   }
 }
 
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// As unit16 above, in FP32.
+template <int T>
+__device__ __forceinline__ void unit16f(float (&x)[4], const float (&l)[16]) {
+  if constexpr (T < 15) {
+    asm volatile("s_nop 1\n\tv_fmac_f32_dpp %0, %0, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %1, %1, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %2, %2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %3, %3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+                 : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3])
+                 : "v"(l[T]), "n"(T));
+    unit16f<T + 1>(x, l);
+  }
+}
+
 // The panel's row permutation (row pos[s] receives the content of slot
-// src[s]; slots 0..nb-1 are rows 0..nb-1) on CB columns of X, then
-// X[0..nb) <- L^{-1} X[0..nb) for those columns (FP32, nb <= 128).  The whole
-// L (unit lower, nb x nb) and every touched row are staged in LDS first, with
-// their loads in flight together; the rows below the top nb are written back
-// permuted and the top nb are solved in LDS, 32-row blocks: one thread per
-// column solves the diagonal block from registers, then all threads update
-// the rows below.
-// LBLK: L kept as its lower 32 x 32 blocks only (under 70 KB of LDS with CB
-// = 16, so the launch fits on a CU beside a trailing-update workgroup).
-template <int CB, bool LBLK>
-__global__ __launch_bounds__(256) void laswp_trsm_kernel(const float* __restrict__ L, int64_t ldl,
-                                                         int nb, float* __restrict__ X,
-                                                         int64_t ldx, int ncols,
-                                                         const int* __restrict__ perm_n,
-                                                         const int* __restrict__ pos,
-                                                         const int* __restrict__ src) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  // (LBLK: the next panel's interchanges and U rows, on the critical path
-  // beside the trailing update's waves: issue priority)
-  if (LBLK) __builtin_amdgcn_s_setprio(3);
-  constexpr int XP = CB + 1;
-  const int nbp = (nb + 31) & ~31, LP = nbp + 1, nbb = nbp / 32;
-  // full: nbp x LP; blocks: (bi, bj), bi >= bj, 32 x 33 each at bi(bi+1)/2 + bj
-  float* Lf = reinterpret_cast<float*>(smem_raw);
-  float* Xs = Lf + (LBLK ? nbb * (nbb + 1) / 2 * 32 * 33 : nbp * LP);  // nbp x XP
-  auto lat = [&](int r, int q) -> float& {
-    if (LBLK) {
-      const int bi = r >> 5, bj = q >> 5;
-      return Lf[((bi * (bi + 1) / 2 + bj) * 32 + (r & 31)) * 33 + (q & 31)];
+// src[s]; slots 0..nb-1 are rows 0..nb-1) on sixteen columns of X per wave,
+// then X[0..nb) <- L^{-1} X[0..nb) for those columns (FP32, nb <= 128): the
+// top rows are read from where they come from, straight into 16 x 16 tiles
+// in registers, every row below is read before any is written, and the solve
+// is trsm_llu64_kernel's (the products of a block summed from zero).  One wave
+// per workgroup, and little LDS: it starts beside the trailing update's
+// workgroups wherever a wave fits.  With L and the touched rows staged in
+// LDS, 32 columns a workgroup and a thread per column: 58 us a launch on
+// average (n = 16384), 25 now; the next panel's 128 columns 22.6 us, 18.4 now.
+__global__ __launch_bounds__(64) void laswp_trsm_kernel(const float* __restrict__ L, int64_t ldl,
+                                                        int nb, float* __restrict__ X,
+                                                        int64_t ldx, int ncols,
+                                                        const int* __restrict__ perm_n,
+                                                        const int* __restrict__ pos,
+                                                        const int* __restrict__ src, int urgent) {
+  // (the next panel's interchanges and U rows, on the critical path beside the
+  // trailing update's waves: issue priority)
+  if (urgent) __builtin_amdgcn_s_setprio(3);
+  constexpr int MAXB = 8, P = 20;  // P: LDS row stride
+  __shared__ __align__(16) float ub[16 * P];
+  const int lane = threadIdx.x, l16 = lane & 15, lk = lane >> 4;
+  const int c0 = blockIdx.x * 16, col = c0 + 4 * lk;
+  const bool whole = c0 + 16 <= ncols;
+  const int nblk = (nb + 15) / 16, nS = *perm_n;
+  auto load = [&](int row) {
+    const float* p = X + (int64_t)row * ldx;
+    if (whole) {
+      const f4u a = *reinterpret_cast<const f4u*>(p + col);
+      return v4f{a.x, a.y, a.z, a.w};
     }
-    return Lf[r * LP + q];
+    v4f a;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) a[r] = p[min(col + r, ncols - 1)];
+    return a;
   };
-  float* buf = Xs + nbp * XP;                      // touched rows x CB
-  int* s_pos = reinterpret_cast<int*>(buf + 2 * nb * CB);
-  int* s_src = s_pos + 2 * nb;
-  const int tid = threadIdx.x;
-  const int c0 = blockIdx.x * CB;
-  const int cw = min(CB, ncols - c0);
-  // L (strictly lower part; zero elsewhere) with the permutation lists, then
-  // the touched rows: every load in flight before the first LDS store (nb <=
-  // 128: at most 64 L words and 2 nb CB / 256 row words per thread)
-  constexpr int NL = 128 * 128 / 256, NR = 2 * 128 * CB / 256;
-  float lv[NL], rv[NR];
+  auto store = [&](int row, v4f a) {
+    float* p = X + (int64_t)row * ldx;
+    if (whole) {
+      *reinterpret_cast<f4u*>(p + col) = f4u{a.x, a.y, a.z, a.w};
+    } else {
 #pragma unroll
-  for (int j = 0; j < NL; ++j) {
-    const int e = tid + 256 * j, r = e / nbp, q = e - r * nbp;
-    lv[j] = (e < nbp * nbp && q < r && r < nb) ? L[(int64_t)r * ldl + q] : 0.f;
-  }
-  const int nS = *perm_n;
-  for (int e = tid; e < nS; e += 256) {
-    s_pos[e] = pos[e];
-    s_src[e] = src[e];
-  }
-  __syncthreads();
+      for (int r = 0; r < 4; ++r)
+        if (col + r < ncols) p[col + r] = a[r];
+    }
+  };
+  // slots 16 i + l16 (the top rows; past nb zero) and nb + 16 i + l16
+  int from[2 * MAXB];
 #pragma unroll
-  for (int j = 0; j < NR; ++j) {
-    const int e = tid + 256 * j, sl = e / CB, c = e - sl * CB;
-    rv[j] = (e < nS * CB && c < cw) ? X[(int64_t)s_pos[sl] * ldx + c0 + c] : 0.f;
+  for (int i = 0; i < 2 * MAXB; ++i) {
+    const int s = (i < MAXB ? 0 : nb) + 16 * (i % MAXB) + l16;
+    from[i] = s < (i < MAXB ? nb : nS) ? src[s] : -1;
   }
 #pragma unroll
-  for (int j = 0; j < NL; ++j) {
-    const int e = tid + 256 * j, r = e / nbp, q = e - r * nbp;
-    if (e < nbp * nbp && (!LBLK || (q >> 5) <= (r >> 5))) lat(r, q) = lv[j];
+  for (int i = 0; i < 2 * MAXB; ++i) from[i] = from[i] >= 0 ? pos[from[i]] : -1;
+  v4f x[MAXB], y[MAXB];
+#pragma unroll
+  for (int i = 0; i < MAXB; ++i) {
+    x[i] = y[i] = v4f{0.f, 0.f, 0.f, 0.f};
+    if (from[i] >= 0) x[i] = load(from[i]);
   }
 #pragma unroll
-  for (int j = 0; j < NR; ++j) {
-    const int e = tid + 256 * j;
-    if (e < nS * CB) buf[e] = rv[j];
-  }
-  __syncthreads();
-  for (int e = tid; e < nbp * CB; e += 256) {
-    const int i = e / CB, c = e - i * CB;
-    Xs[i * XP + c] = i < nb ? buf[s_src[i] * CB + c] : 0.f;
-  }
-  for (int e = nb * CB + tid; e < nS * CB; e += 256) {
-    const int sl = e / CB, c = e - sl * CB;
-    if (c < cw) X[(int64_t)s_pos[sl] * ldx + c0 + c] = buf[s_src[sl] * CB + c];
-  }
-  __syncthreads();
-  for (int b = 0; b < nb; b += 32) {
-    if constexpr (LBLK) {
-      // (the critical-path instance) the diagonal block by substitution with
-      // lanes over rows: a wave takes two columns (lanes 0..31 and 32..63,
-      // row i = lane % 32), each step's solved value broadcast by readlane
-      // (the same operations in the same order as the per-column loop below,
-      // without its dependent chain of 496 FMAs)
-      for (int cp = 2 * (tid >> 6); cp < CB; cp += 2 * 4) {
-        const int lane = tid & 63, i = lane & 31, c = cp + (lane >> 5);
-        float x = c < CB ? Xs[(b + i) * XP + c] : 0.f;
+  for (int i = 0; i < MAXB; ++i)
+    if (from[MAXB + i] >= 0) y[i] = load(from[MAXB + i]);
 #pragma unroll
-        for (int t = 0; t < 31; ++t) {
-          const float lo = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), t));
-          const float hi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 32 + t));
-          const float xt = lane < 32 ? lo : hi;
-          if (i > t) x -= lat(b + i, b + t) * xt;
+  for (int i = 0; i < MAXB; ++i)
+    if (from[MAXB + i] >= 0) store(pos[nb + 16 * i + l16], y[i]);
+  // the next diagonal block's row, requested a block ahead
+  float d[16];
+  auto load_diag = [&](int b) {
+    const float* p = L + (int64_t)min(16 * b + l16, nb - 1) * ldl + 16 * b;
+    if (16 * b + 16 <= nb) {
+#pragma unroll
+      for (int k = 0; k < 16; k += 4) {
+        const f4u a = *reinterpret_cast<const f4u*>(p + k);
+        d[k] = a.x;
+        d[k + 1] = a.y;
+        d[k + 2] = a.z;
+        d[k + 3] = a.w;
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) d[k] = p[min(k, nb - 1 - 16 * b)];
+    }
+  };
+  load_diag(0);
+#pragma unroll 1
+  for (int b = 0; b < nblk; ++b) {
+    float l[16];
+    f4u t[MAXB];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) l[k] = k < l16 && 16 * b + l16 < nb ? -d[k] : 0.f;
+#pragma unroll
+    for (int i = 1; i < MAXB; ++i)
+      if (i > b && i < nblk)  // (block b is whole)
+        t[i] = *reinterpret_cast<const f4u*>(L + (int64_t)min(16 * i + l16, nb - 1) * ldl +
+                                             16 * b + 4 * lk);
+    if (b + 1 < nblk) load_diag(b + 1);
+    float v[4], v0[4];
+#pragma unroll
+    for (int i = 0; i < MAXB; ++i)
+      if (i == b) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = x[i][r];
+      }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v0[r] = v[r];
+    unit16f<0>(v, l);
+    // (as in trsm_llu64_kernel: not finite, again with the rows above masked)
+    const float sum = (v[0] - v[0]) + (v[1] - v[1]) + ((v[2] - v[2]) + (v[3] - v[3]));
+    if (__ballot(!(sum == 0.f))) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = v0[r];
+#pragma unroll
+      for (int k = 0; k < 15; ++k)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float z = __shfl(v[r], (lane & 48) + k);
+          v[r] = l16 > k && 16 * b + l16 < nb ? fmaf(l[k], z, v[r]) : v[r];
         }
-        if (c < CB) Xs[(b + i) * XP + c] = x;
-      }
-    } else if (tid < CB) {
-      float x[32];
-#pragma unroll
-      for (int i = 0; i < 32; ++i) x[i] = Xs[(b + i) * XP + tid];
-#pragma unroll
-      for (int i = 1; i < 32; ++i) {
-        float acc = x[i];
-#pragma unroll
-        for (int q = 0; q < i; ++q) acc -= lat(b + i, b + q) * x[q];
-        x[i] = acc;
-      }
-#pragma unroll
-      for (int i = 0; i < 32; ++i) Xs[(b + i) * XP + tid] = x[i];
     }
-    __syncthreads();
-    for (int e = tid; e < (nbp - b - 32) * CB; e += 256) {
-      const int i = b + 32 + e / CB, c = e % CB;
-      float acc = 0.f;
+    if (16 * b + l16 < nb) store(16 * b + l16, v4f{v[0], v[1], v[2], v[3]});
+    if (b + 1 == nblk) break;
+    *reinterpret_cast<v4f*>(ub + l16 * P + 4 * lk) = v4f{-v[0], -v[1], -v[2], -v[3]};
+    asm volatile("" ::: "memory");  // a wave's LDS accesses execute in order
+    float u[4];
 #pragma unroll
-      for (int q = 0; q < 32; ++q) acc += lat(i, b + q) * Xs[(b + q) * XP + c];
-      Xs[i * XP + c] -= acc;
-    }
-    __syncthreads();
-  }
-  for (int e = tid; e < nb * CB; e += 256) {
-    const int i = e / CB, c = e - i * CB;
-    if (c < cw) X[(int64_t)i * ldx + c0 + c] = Xs[i * XP + c];
+    for (int j = 0; j < 4; ++j) u[j] = ub[(4 * lk + j) * P + l16];
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int i = 1; i < MAXB; ++i)
+      if (i > b && i < nblk) {
+        v4f e = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          e = __builtin_amdgcn_mfma_f32_16x16x4f32(u[j], t[i][j], e, 0, 0, 0);
+        x[i] += e;
+      }
   }
 }
 
@@ -511,32 +539,14 @@ int trsm_llu_rowmajor(hipStream_t s, const T* L, int64_t ldl, int nb, T* X, int6
 // the U rows of those columns in one launch (FP32, nb <= 128).
 int laswp_trsm_rowmajor(hipStream_t s, const float* L, int64_t ldl, int nb, float* X, int64_t ldx,
                         int ncols, const int* perm_n, const int* pos, const int* src,
-                        bool compact) {
+                        bool urgent) {
   if (ncols <= 0 || nb <= 0) return kOk;
   if (nb > 128) {
     set_error("laswp_trsm: panel width %d > 128", nb);
     return kErrUnsupported;
   }
-  const size_t nbp = (size_t)((nb + 31) & ~31), nbb = nbp / 32;
-  auto lds_of = [&](int cb, bool lblk) {
-    return sizeof(float) * ((lblk ? nbb * (nbb + 1) / 2 * 32 * 33 : nbp * (nbp + 1)) +
-                            nbp * (cb + 1) + 2 * (size_t)nb * cb) +
-           sizeof(int) * 4 * (size_t)nb;
-  };
-  static bool attr_set = false;
-  if (!attr_set) {
-    EAMD_HIP(hipFuncSetAttribute((const void*)laswp_trsm_kernel<32, false>,
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
-    EAMD_HIP(hipFuncSetAttribute((const void*)laswp_trsm_kernel<4, true>,
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
-    attr_set = true;
-  }
-  if (compact)
-    hipLaunchKernelGGL((laswp_trsm_kernel<4, true>), dim3(ceil_div(ncols, 4)), dim3(256),
-                       lds_of(4, true), s, L, ldl, nb, X, ldx, ncols, perm_n, pos, src);
-  else
-    hipLaunchKernelGGL((laswp_trsm_kernel<32, false>), dim3(ceil_div(ncols, 32)), dim3(256),
-                       lds_of(32, false), s, L, ldl, nb, X, ldx, ncols, perm_n, pos, src);
+  hipLaunchKernelGGL(laswp_trsm_kernel, dim3(ceil_div(ncols, 16)), dim3(64), 0, s, L, ldl, nb, X,
+                     ldx, ncols, perm_n, pos, src, urgent ? 1 : 0);
   EAMD_HIP(hipGetLastError());
   return kOk;
 }
