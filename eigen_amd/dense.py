@@ -89,7 +89,9 @@ def gemm(A, B, C_=None, alpha=1.0, beta=0.0, transa="N", transb="N"):
     k = A.shape[1] if transa == "N" else A.shape[0]
     n = B.shape[1] if transb == "N" else B.shape[0]
     if C_ is None:
-        C_ = colmajor(torch.zeros(m, n, dtype=torch.float64, device=A.device))
+        # column-major and not cleared: beta = 0 writes every element (k = 0
+        # clears C too); a fill and a copy were half of a small call's time
+        C_ = torch.empty(n, m, dtype=torch.float64, device=A.device).t()
         beta = 0.0
     else:
         C_ = colmajor(C_, torch.float64)
