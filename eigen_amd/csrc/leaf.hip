@@ -960,7 +960,9 @@ namespace {
 // and scaling per wave beside its FMAs, so a lone wave of each SIMD with four
 // rows per lane issued one every six cycles and waited on LDS in between
 // (1024 rows in four waves: 2000 cycles a column; 512 in two: 1650; 256 in
-// one: 1350).  The registers stay within what one of the trailing update's
+// one: 1350; now about 1600, 1300 and 1100).  16384 rows: local and final
+// round 30 + 51 us before (512-row groups, 1024 candidates), 34 + 30 now;
+// 4096 rows 24 + 50 before, 18 + 30 now.  The registers stay within what one of the trailing update's
 // workgroups gives back when it ends (272 per SIMD): a round that needed the
 // room of two would wait until the update drains.
 template <int CAP>
@@ -1453,8 +1455,8 @@ __global__ __launch_bounds__(256) void tsl_apply_kernel(float* __restrict__ P, i
 // top rows.  Then each wave updates 16 rows by FP32 matrix products, C
 // requested at the start.  The solves' serial chains bound it (500 dependent
 // steps, L11\U11 read from LDS four values at a time); with four threads a
-// row, each solving it again and reading an LDS word per FMA, it took 23 us for
-// 16384 rows.
+// row, each solving it again and reading an LDS word per FMA, it took 23 us on
+// average over the panels of n = 16384, and 15 now.
 constexpr int kApplyRows = 64;
 constexpr int kFuseRestMax = 96;  // panel columns right of a fused leaf (panels <= 128)
 __global__ __launch_bounds__(256) void tsl_apply_rest_kernel(float* __restrict__ P, int64_t ldp,
